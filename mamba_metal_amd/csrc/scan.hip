@@ -21,7 +21,9 @@
 //     predecessor segment's flag, reads the carried fp32 state, scans its segment,
 //     writes the state and raises its own flag.  Every predecessor was claimed earlier
 //     by a resident workgroup, so the wait always ends; the spin is bounded anyway.
-//     Segment-major units balance any number of chains over the CUs.  With few chains
+//     Segment-major units balance any number of chains over the CUs.  With fewer chains
+//     the scan runs with time across the lanes instead (scan_lanes.hip, where its plan()
+//     takes the call), and between the two
 //     the split mode (see Mode) replaces the hand-off by segment summaries; its units
 //     never wait, so its workgroups take them by a static stride (unit = workgroup +
 //     k * grid) instead of the ticket atomic, which all workgroups of a short launch
@@ -37,7 +39,7 @@
 //     = exp2(delta2 * A); the packed B carries the matching factor ln(2).
 #include <algorithm>
 
-#include "mm_common.h"
+#include "scan_common.h"
 
 namespace mm {
 namespace scan {
@@ -249,20 +251,6 @@ struct Vec<DT, 2> {
   using T = typename Ty<DT>::T;
   typedef T type __attribute__((ext_vector_type(2)));
 };
-
-// delta2 = delta' * log2(e), delta' = x <= cut ? softplus(x) : x.  cut is the reference's
-// softplus cutoff 20 when delta_softplus is on, NaN when it is off (every comparison with
-// NaN is false: delta' = x), so the flag costs no select of its own.  fp32 inputs keep
-// log1p accuracy; fp16/bf16 inputs (whose own rounding is 2^-11 / 2^-8) use
-// log2(1 + 2^m) directly.
-template <int DT>
-__device__ __forceinline__ float delta_log2(float x, float cut) {
-  const float m = x * kLog2e;
-  float l;
-  if constexpr (DT == MM_F32) l = log1p_exp(x) * kLog2e;
-  else l = log2_hw(1.0f + exp2_hw(m));
-  return x <= cut ? l : m;
-}
 
 // ---------------------------------------------------------------------------
 template <int DT, int LAYOUT, int SPL, int G, bool VEC, int MODE, int CPW>
@@ -1068,6 +1056,13 @@ int fwd(const mm_scan_params* a, void* stream, bool chained_min_ok) {
     return fail(MM_ERR_WORKSPACE, "workspace of %zu bytes required, got %zu (%s)", need,
                 a->workspace_bytes, a->workspace ? "too small" : "NULL");
   if (!aligned(a->workspace, 256)) return fail(MM_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+
+  const size_t sum_bytes = a->workspace_bytes >= w.total ? w.total - w.sum : 0;
+  if (lscan::preferred(a, sum_bytes)) {
+    char* const wsp = static_cast<char*>(a->workspace);
+    return lscan::launch(a, reinterpret_cast<int*>(wsp), reinterpret_cast<float*>(wsp + w.sum), sum_bytes,
+                         stream);
+  }
 
   Params p;
   p.A = a->A;

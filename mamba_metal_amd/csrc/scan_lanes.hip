@@ -1,0 +1,703 @@
+// Selective scan with time across the lanes of a wave: mm_selective_scan_fwd[_strided] for scans
+// of few channels (see plan), where scan.hip's chains -- one lane per channel, walking time --
+// are too few to fill the chip.  Semantics as in scan.hip.
+//
+// A wave takes one channel and walks its sequence in chunks of 512 steps, 8 consecutive steps
+// per lane.  Per state: the lane's decays a = exp2(delta2 A) and inputs b = delta' u B are
+// computed once and kept in registers; the lane's end state from zero (one fma per step); an
+// inclusive scan of the lanes' (decay, end state) pairs through DPP (a lane's decay is
+// exp2 of A times its sum of delta2, so it is not multiplied up); then the recurrence once more
+// from the lane's true start state, and y += C h.  Seven VALU slots per (channel, state, step)
+// -- one of six more than the sequential walk -- plus ~30 per state and chunk for the lane scan,
+// and y needs no sum over waves.  B and C are staged in LDS as fp32, eight states at a time
+// (the next group's loads in flight during this one's arithmetic), shared by the workgroup's
+// channels.  SW > 1 shares a channel's states among SW waves, for launches that would leave
+// SIMDs idle; with few channels and a long sequence time is split as well: a first launch
+// (SUM) leaves every segment's end state from zero and its sum of delta2, and the second folds
+// its predecessors' with one more lane scan.
+//
+// What bounds it: VALU issue (at B=4 D=1536 L=4096 fp16, 12 instructions and 13.9 issue slots
+// per update, 98% of the VALU's cycles busy), against 9.6-12 slots for scan.hip where that one's
+// chains fill the chip, and its 14-40 where they do not.  Tried and not kept: 16 steps per
+// lane (11 slots, but two waves per SIMD instead of four: B=4 D=1536 L=4096 149 -> 180 us), two
+// states interleaved per wave (149 -> 186), the next state's LDS reads ahead (149 -> 151).
+#include <algorithm>
+#include <type_traits>
+
+#include "scan_common.h"
+
+namespace mm {
+namespace lscan {
+
+constexpr int kTL = 8;                 // steps per lane and chunk
+constexpr int kChunk = 64 * kTL;       // steps per chunk
+constexpr int kNG = 8;                 // states of B and C staged at a time
+constexpr int kItems = kNG * kChunk / 8;  // 8-element items of a staged tensor
+constexpr int kXcds = 8;
+constexpr int kMaxSeg = 64;  // a wave folds its segment's predecessors, one per lane
+
+// kTime: u, delta, z, y and B, C contiguous along time.  kRows: u, delta, z, y contiguous along
+// channels (a multiple of 8), B, C along states (a multiple of 8).
+enum Layout { kTime = 0, kRows = 1 };
+
+struct Params {
+  const void* u;
+  const void* delta;
+  const void* z;
+  void* y;
+  const float* A;
+  const float* D;
+  const void* B;
+  const void* C;
+  float* state_out;
+  float* sum;    // [batch][dim][dstate + 1][nseg] segment summaries: end states, then sum of delta2
+  int* ctl;
+  int64_t us0, us1, us2, ds0, ds1, ds2, zs0, zs1, zs2, ys0, ys1, ys2;
+  int64_t Bs0, Bs1, Bs2, Cs0, Cs1, Cs2, As0, As1, Ds;
+  int32_t dim, dstate, seqlen, nseg, seg_chunks;
+  float softplus_cut;
+};
+
+// N elements at any element-aligned address (the hardware takes unaligned global accesses), so
+// odd lengths and strides need no path of their own.
+template <int DT, int N>
+struct Run {
+  typedef typename Ty<DT>::T V __attribute__((ext_vector_type(N)));
+  typedef typename Ty<DT>::T U __attribute__((ext_vector_type(N), aligned(sizeof(typename Ty<DT>::T))));
+};
+
+// Value of x in another lane through DPP; lanes without a source get `old`.
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ float dpp_or(float old, float x) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), CTRL, ROWS, 0xF, false));
+}
+// ... get 0.
+template <int CTRL>
+__device__ __forceinline__ float dpp_or0(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+constexpr int kRowShr = 0x110;   // + n: lane i of a 16-lane row takes lane i - n
+constexpr int kWaveShr1 = 0x138; // lane i takes lane i - 1
+constexpr int kBcast15 = 0x142;  // rows 1 and 3 take the last lane of the row before
+constexpr int kBcast31 = 0x143;  // rows 2 and 3 take lane 31
+
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// LDS rows of one state's B or C: the four steps 4q .. 4q + 3 of every lane lie together, so a
+// lane reads its steps as float4s next to its neighbours'.  Each q's block is rotated, so
+// that 64 consecutive steps lie on distinct banks when they are written one by one.
+__device__ __forceinline__ int lds_lane(int lane, int q) { return q * 256 + ((lane * 4 + q * 32) & 255); }
+__device__ __forceinline__ int lds_pos(int t) { return lds_lane(t / kTL, (t % kTL) >> 2) + (t & 3); }
+
+// Inclusive prefix sums over the lanes: within each 16-lane row, within each half, whole.
+__device__ __forceinline__ void prefix(float s, float& row, float& half, float& all) {
+  s += dpp_or0<kRowShr + 1>(s);
+  s += dpp_or0<kRowShr + 2>(s);
+  s += dpp_or0<kRowShr + 4>(s);
+  s += dpp_or0<kRowShr + 8>(s);
+  row = s;
+  half = s + dpp_or<kBcast15, 0xA>(0.0f, s);
+  all = half + dpp_or<kBcast31, 0xC>(0.0f, half);
+}
+
+// Inclusive scan over the lanes of the recurrence's (decay, state) pairs: on entry P and h are
+// a lane's decay over its own steps and its end state from a zero start; on return h is the
+// end state from the start of the wave.  pr and ph: the lane's decay since the start of its
+// 16-lane row and of its half-wave.  Lanes without a source in a row step read decay and state
+// 0 (they are complete by then).  Each s_nop covers the two wait states between a VALU write
+// of a register and its read through DPP.
+__device__ __forceinline__ void lane_scan(float& P, float& h, float pr, float ph) {
+  asm volatile(
+      "s_nop 1\n\t"
+      "v_fmac_f32_dpp %1, %1, %0 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "s_nop 0\n\t"
+      "v_fmac_f32_dpp %1, %1, %0 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "s_nop 0\n\t"
+      "v_fmac_f32_dpp %1, %1, %0 row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "s_nop 0\n\t"
+      "v_fmac_f32_dpp %1, %1, %0 row_shr:8 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "s_nop 1\n\t"
+      "v_fmac_f32_dpp %1, %1, %2 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_fmac_f32_dpp %1, %1, %3 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+      "s_nop 1"
+      : "+v"(P), "+v"(h)
+      : "v"(pr), "v"(ph));
+}
+
+// B and C of NG states of a chunk on their way to LDS rows of fp32, zero past the sequence's
+// end and past the last state: one vector of 8 steps of a state (kTime) or of 8 states of a
+// step (kRows) per thread and tensor.
+
+template <int DT, int LAYOUT, int NT>
+struct Stage {
+  using T = typename Ty<DT>::T;
+  using V = typename Run<DT, 8>::V;
+  using U = typename Run<DT, 8>::U;
+  static constexpr int kPer = kChunk / 8;         // kTime: 8-step items of a state
+  static constexpr bool kSplit = NT == 2 * kItems;  // half the threads take B, half C
+  static_assert(NT == kItems || kSplit, "one item of B and of C per thread, or of one of them");
+  V v[kSplit ? 1 : 2];
+  const T* ptr[kSplit ? 1 : 2];  // this thread's item of state group 0 and step 0
+  int64_t sn, st;                // its tensor's strides along states and time (kSplit)
+
+  __device__ __forceinline__ int item(int tid) const { return kSplit ? tid & (kItems - 1) : tid; }
+
+  __device__ __forceinline__ void init(const Params& p, int64_t bat, int tid) {
+    const T* const pb = static_cast<const T*>(p.B) + bat * p.Bs0;
+    const T* const pc = static_cast<const T*>(p.C) + bat * p.Cs0;
+    const int i = item(tid);
+    if constexpr (kSplit) {
+      const bool isb = __builtin_amdgcn_readfirstlane(tid) < kItems;  // whole waves
+      sn = isb ? p.Bs1 : p.Cs1;
+      st = isb ? p.Bs2 : p.Cs2;
+      ptr[0] = (isb ? pb : pc) + (LAYOUT == kTime ? (i / kPer) * sn + 8 * (i % kPer) : i * st);
+    } else {
+      ptr[0] = pb + (LAYOUT == kTime ? (i / kPer) * p.Bs1 + 8 * (i % kPer) : i * p.Bs2);
+      ptr[1] = pc + (LAYOUT == kTime ? (i / kPer) * p.Cs1 + 8 * (i % kPer) : i * p.Cs2);
+    }
+  }
+
+  __device__ __forceinline__ void load(const Params& p, bool with_c, int g0, int t0, int tid) {
+    const bool full = t0 + kChunk <= p.seqlen && g0 + kNG <= p.dstate;
+#pragma unroll
+    for (int x = 0; x < (kSplit ? 1 : 2); ++x) {
+      if (x == 1 && !with_c) break;
+      const int64_t s1 = kSplit ? sn : x ? p.Cs1 : p.Bs1, s2 = kSplit ? st : x ? p.Cs2 : p.Bs2;
+      int64_t o;
+      if constexpr (LAYOUT == kTime) {
+        o = g0 * s1 + t0;
+        if (!full) {
+          // states past the last read the last one, the sequence's last vector lies 8 steps
+          // before its end
+          const int n = item(tid) / kPer, t = 8 * (item(tid) % kPer);
+          o += static_cast<int64_t>(std::min(n, p.dstate - 1 - g0) - n) * s1 + (std::min(t, p.seqlen - 8 - t0) - t);
+        }
+      } else {
+        int dt = t0;
+        if (!full) dt = t0 + item(tid) < p.seqlen ? dt : -item(tid);  // steps past the end read step 0
+        o = dt * s2 + g0;
+      }
+      v[x] = *reinterpret_cast<const U*>(ptr[x] + o);
+    }
+  }
+
+  __device__ __forceinline__ void store(const Params& p, bool with_c, int g0, int t0, int tid,
+                                        float (*sb)[kChunk], float (*sc)[kChunk]) const {
+    const bool full = t0 + kChunk <= p.seqlen && g0 + kNG <= p.dstate;
+#pragma unroll
+    for (int x = 0; x < (kSplit ? 1 : 2); ++x) {
+      float(*const dst)[kChunk] = kSplit ? (__builtin_amdgcn_readfirstlane(tid) < kItems ? sb : sc) : x ? sc : sb;
+      if (!with_c && dst == sc) break;
+      if constexpr (LAYOUT == kTime) {
+        const int n = item(tid) / kPer, t = 8 * (item(tid) % kPer);
+        if (full) {
+#pragma unroll
+          for (int q = 0; q < 8; q += 4)
+            *reinterpret_cast<float4*>(&dst[n][lds_pos(t + q)]) = make_float4(
+                Ty<DT>::f(v[x][q]), Ty<DT>::f(v[x][q + 1]), Ty<DT>::f(v[x][q + 2]), Ty<DT>::f(v[x][q + 3]));
+        } else {
+          // elements go to their own steps (the clamped vector's first ones once more, with the
+          // same values); steps past the end are zeroed.  tt is opaque: these positions are not
+          // worth registers in every chunk.
+          const bool nin = g0 + n < p.dstate;
+          int tt = t;
+          asm volatile("" : "+v"(tt));
+          const int back = std::max(t0 + tt - (p.seqlen - 8), 0);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            if (t0 + tt < p.seqlen && tt - back + k >= 0)
+              dst[n][lds_pos(tt - back + k)] = nin ? Ty<DT>::f(v[x][k]) : 0.0f;
+            if (t0 + tt + k >= p.seqlen) dst[n][lds_pos(tt + k)] = 0.0f;
+          }
+        }
+      } else {
+        const int t = item(tid), pos = lds_pos(t);
+        const bool in = full || t0 + t < p.seqlen;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) dst[k][pos] = in ? Ty<DT>::f(v[x][k]) : 0.0f;
+      }
+    }
+  }
+};
+
+// CH channels per workgroup, each on SW waves that share its states.  kDirect: a lane loads and
+// stores its own steps; otherwise every thread owns 8 / SW elements of the chunk (steps of a
+// channel, or channels of a step) and they pass through an LDS tile.
+template <int DT, int LAYOUT, bool SUM, int CH, int SW>
+__global__ __launch_bounds__(64 * CH * SW, 4) void lane_scan_kernel(const Params p) {
+  using T = typename Ty<DT>::T;
+  constexpr int NT = 64 * CH * SW;
+  constexpr bool kDirect = LAYOUT == kTime && SW == 1;
+  static_assert(LAYOUT == kTime || NT % kChunk == 0, "threads in whole chunks");
+  constexpr int E = 8 / SW;          // elements of a thread per chunk and tensor
+  constexpr int kStates = kNG / SW;  // states of a wave in a staged group
+  using V = typename Run<DT, E>::V;
+  using U = typename Run<DT, E>::U;
+
+  __shared__ __attribute__((aligned(16))) float s_b[kNG][kChunk];
+  __shared__ __attribute__((aligned(16))) float s_c[SUM ? 1 : kNG][kChunk];
+  // the tile: delta2 and delta' * u, then the partial y's of the waves of a channel
+  constexpr int kAreas = kDirect ? 0 : SUM || SW <= 2 ? 2 : SW;
+  __shared__ __attribute__((aligned(16))) float s_x[kAreas > 0 ? kAreas : 1][kDirect ? 1 : CH][kDirect ? 4 : kChunk];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wch = wave % CH, part = wave / CH;
+  // Workgroups go to the XCDs (each with an L2 of its own) in turn.  Neighbouring channel groups
+  // share the 128-byte lines of channel-contiguous tensors, so each XCD takes a run of them.
+  int unit;
+  {
+    const int n = gridDim.x, x = blockIdx.x % kXcds, k = blockIdx.x / kXcds;
+    unit = x * (n / kXcds) + std::min(x, n % kXcds) + k;
+  }
+  const int ncg = (p.dim + CH - 1) / CH;
+  const int ch0 = unit % ncg * CH;
+  const int seg = unit / ncg % p.nseg;
+  const int64_t b = unit / ncg / p.nseg;
+  const int ch = ch0 + wch;
+  const bool chok = ch < p.dim;
+  const int c = chok ? ch : p.dim - 1;  // waves past dim repeat the last channel, unstored
+  const bool has_z = p.z != nullptr;
+  if (!SUM && unit == 0 && tid == 0) p.ctl[1] = 0;  // the call's status
+
+  // lane n holds the channel's A[n] and the carried state n
+  const float Al = lane < p.dstate ? p.A[c * p.As0 + lane * p.As1] : 0.0f;
+  const bool mine = SW == 1 || lane % kNG / kStates == part;  // whether this wave has state n = lane
+  const bool Apos = __any(Al > 0.0f);
+  const bool may_grow = Apos || p.softplus_cut != p.softplus_cut;
+  float Amax = fabsf(Al);
+  for (int m = 32; m > 0; m >>= 1) Amax = fmaxf(Amax, lane_xor(Amax, m));
+  float carry = 0.0f;
+  float dsum = 0.0f;  // SUM: delta2 over the segment
+
+  if (!SUM && seg > 0) {
+    // carry into the segment: predecessors' end states decayed over what lies between.  Lane i
+    // takes segment seg - 1 - i; its distance is the sum of delta2 of the segments after.
+    const float* const sm = p.sum + (b * p.dim + c) * (p.dstate + 1) * static_cast<int64_t>(p.nseg);
+    const int j = lane < seg ? seg - 1 - lane : 0;
+    const float ds = lane < seg ? sm[static_cast<int64_t>(p.dstate) * p.nseg + j] : 0.0f;
+    float r, hf, all;
+    prefix(ds, r, hf, all);
+    const float w = dpp_or<kWaveShr1>(0.0f, all);
+    const bool grows = Apos || __any(ds < 0.0f);  // see `serial` below
+    for (int g0 = 0; g0 < p.dstate; g0 += kNG) {
+      float v[kStates];
+#pragma unroll
+      for (int k = 0; k < kStates; ++k) {
+        const int n = g0 + part * kStates + k;
+        v[k] = (lane < seg && n < p.dstate) ? sm[static_cast<int64_t>(n) * p.nseg + j] : 0.0f;
+      }
+#pragma unroll
+      for (int k = 0; k < kStates; ++k) {
+        const int n = g0 + part * kStates + k;
+        const float An = lane_value(Al, n & 63);
+        float hin;
+        if (grows) {
+          hin = 0.0f;
+          for (int i = seg - 1; i >= 0; --i) {
+            // a segment's factor may overflow where its product with a small state does not: in
+            // sixteen steps (and not at all on a zero state)
+            const float f = exp2_decay<DT>(An * lane_value(ds, i) * 0.0625f);
+            float g = hin;
+            for (int r = 0; r < 16; ++r) g *= f;
+            hin = (hin == 0.0f ? 0.0f : g) + lane_value(v[k], i);
+          }
+        } else {
+          float vr, vh, va;
+          prefix(v[k] * exp2_decay<DT>(w * An), vr, vh, va);
+          hin = lane_value(va, 63);
+        }
+        carry = lane == n ? hin : carry;
+      }
+    }
+  }
+
+  const int nch = (p.seqlen + kChunk - 1) / kChunk;
+  const int c_begin = seg * p.seg_chunks;
+  const int c_end = c_begin + p.seg_chunks < nch ? c_begin + p.seg_chunks : nch;
+
+  const T* const up = static_cast<const T*>(p.u) + b * p.us0;
+  const T* const dp = static_cast<const T*>(p.delta) + b * p.ds0;
+  const T* const zp = has_z ? static_cast<const T*>(p.z) + b * p.zs0 : up;
+  const int64_t zs1 = has_z ? p.zs1 : p.us1, zs2 = has_z ? p.zs2 : p.us2;
+  T* const yp = static_cast<T*>(p.y) + b * p.ys0;
+  // this thread's elements: from step et of the chunk (and, by rows, from channel ch0 + ec)
+  const int et = LAYOUT == kTime ? (kDirect ? lane * kTL : part * 64 * E + lane * E) : tid & (kChunk - 1);
+  const int ec = LAYOUT == kTime ? wch : tid / kChunk * E;
+  float Dv[LAYOUT == kTime ? 1 : E];
+#pragma unroll
+  for (int k = 0; k < (LAYOUT == kTime ? 1 : E); ++k)
+    Dv[k] = (!SUM && p.D) ? p.D[(ch0 + ec + k < p.dim ? ch0 + ec + k : p.dim - 1) * p.Ds] : 0.0f;
+
+  auto load = [&](const T* base, int64_t s1, int64_t s2, int t0, V& v) __attribute__((always_inline)) {
+    if constexpr (LAYOUT == kTime) {
+      const T* const r = base + c * s1 + t0 + et;
+      if (t0 + kChunk <= p.seqlen) {
+        v = *reinterpret_cast<const U*>(r);
+      } else {
+#pragma unroll
+        for (int k = 0; k < E; ++k) v[k] = t0 + et + k < p.seqlen ? r[k] : Ty<DT>::from(0.0f);
+      }
+    } else {
+      v = *reinterpret_cast<const U*>(base + (t0 + et < p.seqlen ? t0 + et : 0) * s2 + ch0 + ec);
+    }
+  };
+  // whether element k of this thread lies inside the sequence (tt: its first step)
+  auto inside = [&](int tt, int k) { return (LAYOUT == kTime ? tt + k : tt) < p.seqlen; };
+
+  V ru, rd, rz, ku;  // the chunk's u, delta, z, and u kept for the skip term
+  Stage<DT, LAYOUT, NT> st;
+  load(up, p.us1, p.us2, c_begin * kChunk, ru);
+  load(dp, p.ds1, p.ds2, c_begin * kChunk, rd);
+  st.init(p, b, tid);
+  st.load(p, !SUM, 0, c_begin * kChunk, tid);
+
+  for (int chunk = c_begin; chunk < c_end; ++chunk) {
+    const int t0 = chunk * kChunk;
+    float d2[kTL], du[kTL], y[kTL];
+    float S, Srow, Shalf;
+    bool serial = false;
+
+    for (int g0 = 0; g0 < p.dstate; g0 += kNG) {
+      const bool last = g0 + kNG >= p.dstate;
+      __syncthreads();  // the staged states and the tile are read
+      st.store(p, !SUM, g0, t0, tid, s_b, s_c);
+      if (g0 == 0) {
+        // this thread's elements: delta2 and delta' * u
+        float ed[E], eu[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+          ed[k] = scan::delta_log2<DT>(Ty<DT>::f(rd[k]), p.softplus_cut);
+          eu[k] = ed[k] * kLn2 * Ty<DT>::f(ru[k]);
+        }
+        if (t0 + kChunk > p.seqlen) {
+          int tt = t0 + et;
+          asm volatile("" : "+v"(tt));  // keeps this a branch
+#pragma unroll
+          for (int k = 0; k < E; ++k) {
+            ed[k] = inside(tt, k) ? ed[k] : 0.0f;  // identity step past the end
+            eu[k] = inside(tt, k) ? eu[k] : 0.0f;
+          }
+        }
+        ku = ru;
+        if constexpr (kDirect) {
+#pragma unroll
+          for (int j = 0; j < kTL; ++j) d2[j] = ed[j], du[j] = eu[j];
+        } else if constexpr (LAYOUT == kTime) {
+          typedef float FV __attribute__((ext_vector_type(E)));
+          FV dv, uv;
+#pragma unroll
+          for (int k = 0; k < E; ++k) dv[k] = ed[k], uv[k] = eu[k];
+          *reinterpret_cast<FV*>(&s_x[0][ec][lds_pos(et)]) = dv;
+          *reinterpret_cast<FV*>(&s_x[1][ec][lds_pos(et)]) = uv;
+        } else {
+          const int pos = lds_pos(et);
+#pragma unroll
+          for (int k = 0; k < E; ++k) {
+            s_x[0][ec + k][pos] = ed[k];
+            s_x[1][ec + k][pos] = eu[k];
+          }
+        }
+      }
+      if (!last) st.load(p, !SUM, g0 + kNG, t0, tid);
+      else if (chunk + 1 < c_end) st.load(p, !SUM, 0, t0 + kChunk, tid);
+      __syncthreads();
+
+      if (g0 == 0) {
+        if constexpr (!kDirect) {
+#pragma unroll
+          for (int q = 0; q < kTL / 4; ++q) {
+            const float4 dv = *reinterpret_cast<const float4*>(&s_x[0][wch][lds_lane(lane, q)]);
+            const float4 uv = *reinterpret_cast<const float4*>(&s_x[1][wch][lds_lane(lane, q)]);
+            d2[4 * q] = dv.x, d2[4 * q + 1] = dv.y, d2[4 * q + 2] = dv.z, d2[4 * q + 3] = dv.w;
+            du[4 * q] = uv.x, du[4 * q + 1] = uv.y, du[4 * q + 2] = uv.z, du[4 * q + 3] = uv.w;
+          }
+        }
+        S = d2[0];
+#pragma unroll
+        for (int j = 1; j < kTL; ++j) S += d2[j];
+        float Sall;
+        prefix(S, Srow, Shalf, Sall);
+        if constexpr (SUM) dsum += lane_value(Sall, 63);
+#pragma unroll
+        for (int j = 0; j < kTL; ++j) y[j] = 0.0f;
+        // Growing states (A > 0, or delta < 0 without the softplus): products of decays may
+        // overflow where the recurrence itself does not, so then the lanes go one by one.
+        serial = false;
+        if (may_grow) {
+          float mag = 0.0f, lo = 0.0f, r, hf, all;
+#pragma unroll
+          for (int j = 0; j < kTL; ++j) {
+            lo = fminf(lo, d2[j]);
+            mag += fabsf(d2[j]);
+          }
+          prefix(mag, r, hf, all);
+          serial = (Apos || __any(lo < 0.0f)) && !(lane_value(all, 63) * Amax < 60.0f);
+        }
+      }
+      if (last) {  // in flight during these states
+        if (!SUM) load(zp, zs1, zs2, t0, rz);
+        if (chunk + 1 < c_end) {
+          load(up, p.us1, p.us2, t0 + kChunk, ru);
+          load(dp, p.ds1, p.ds2, t0 + kChunk, rd);
+        }
+      }
+
+      const int n_end = std::min((part + 1) * kStates, p.dstate - g0);
+#pragma unroll 1
+      for (int n = part * kStates; n < n_end; ++n) {
+        const float A = lane_value(Al, g0 + n), cin = lane_value(carry, g0 + n);
+        float a[kTL], bb[kTL];
+#pragma unroll
+        for (int q = 0; q < kTL / 4; ++q) {
+          const float4 v = *reinterpret_cast<const float4*>(&s_b[n][lds_lane(lane, q)]);
+          bb[4 * q] = du[4 * q] * v.x;
+          bb[4 * q + 1] = du[4 * q + 1] * v.y;
+          bb[4 * q + 2] = du[4 * q + 2] * v.z;
+          bb[4 * q + 3] = du[4 * q + 3] * v.w;
+        }
+#pragma unroll
+        for (int j = 0; j < kTL; ++j) a[j] = exp2_decay<DT>(d2[j] * A);
+        float hx, hend;  // the state before this lane's steps, and at the chunk's end
+        if (!serial) {
+          float h = lane == 0 ? cin : 0.0f;
+#pragma unroll
+          for (int j = 0; j < kTL; ++j) h = __builtin_fmaf(a[j], h, bb[j]);
+          float P = exp2_decay<DT>(S * A);
+          lane_scan(P, h, exp2_decay<DT>(Srow * A), exp2_decay<DT>(Shalf * A));
+          hx = dpp_or<kWaveShr1>(cin, h);
+          hend = lane_value(h, 63);
+        } else {
+          hx = hend = cin;
+          for (int l = 0; l < 64; ++l) {
+            hx = lane == l ? hend : hx;
+            float v = hend;
+#pragma unroll
+            for (int j = 0; j < kTL; ++j) v = __builtin_fmaf(a[j], v, bb[j]);
+            hend = lane_value(v, l);
+          }
+        }
+        carry = lane == g0 + n ? hend : carry;
+        if constexpr (!SUM) {
+#pragma unroll
+          for (int q = 0; q < kTL / 4; ++q) {
+            const float4 v = *reinterpret_cast<const float4*>(&s_c[n][lds_lane(lane, q)]);
+            const float cc[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              hx = __builtin_fmaf(a[4 * q + j], hx, bb[4 * q + j]);
+              y[4 * q + j] = __builtin_fmaf(hx, cc[j], y[4 * q + j]);
+            }
+          }
+        }
+      }
+    }
+
+    if constexpr (SUM) continue;
+    // ---- skip term, gate and store ----
+    float ey[E];
+    if constexpr (kDirect) {
+#pragma unroll
+      for (int k = 0; k < E; ++k) ey[k] = y[k];
+    } else {
+      __syncthreads();  // the tile's delta2 and delta' * u are read
+#pragma unroll
+      for (int q = 0; q < kTL / 4; ++q)
+        *reinterpret_cast<float4*>(&s_x[part][wch][lds_lane(lane, q)]) =
+            make_float4(y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]);
+      __syncthreads();
+      const int pos = lds_pos(et);
+#pragma unroll
+      for (int k = 0; k < E; ++k) {
+        ey[k] = LAYOUT == kTime ? s_x[0][ec][pos + k] : s_x[0][ec + k][pos];
+#pragma unroll
+        for (int w = 1; w < SW; ++w) ey[k] += LAYOUT == kTime ? s_x[w][ec][pos + k] : s_x[w][ec + k][pos];
+      }
+    }
+    V o;
+#pragma unroll
+    for (int k = 0; k < E; ++k) ey[k] = __builtin_fmaf(Dv[LAYOUT == kTime ? 0 : k], Ty<DT>::f(ku[k]), ey[k]);
+    if (has_z) {
+#pragma unroll
+      for (int k = 0; k < E; ++k) o[k] = Ty<DT>::from(ey[k] * silu_f(Ty<DT>::f(rz[k])));
+    } else {
+#pragma unroll
+      for (int k = 0; k < E; ++k) o[k] = Ty<DT>::from(ey[k]);
+    }
+    if constexpr (LAYOUT == kTime) {
+      T* const r = yp + c * p.ys1 + t0 + et;
+      if (!chok) continue;
+      if (t0 + kChunk <= p.seqlen) {
+        *reinterpret_cast<U*>(r) = o;
+      } else {
+#pragma unroll
+        for (int k = 0; k < E; ++k)
+          if (t0 + et + k < p.seqlen) r[k] = o[k];
+      }
+    } else if (t0 + et < p.seqlen) {
+      *reinterpret_cast<U*>(yp + (t0 + et) * p.ys2 + ch0 + ec) = o;
+    }
+  }
+
+  if (!chok || !mine) return;
+  if constexpr (SUM) {
+    float* const sm = p.sum + (b * p.dim + c) * (p.dstate + 1) * static_cast<int64_t>(p.nseg) + seg;
+    if (lane < p.dstate) sm[static_cast<int64_t>(lane) * p.nseg] = carry;
+    if (lane == 0) sm[static_cast<int64_t>(p.dstate) * p.nseg] = dsum;
+  } else if (p.state_out != nullptr && seg + 1 == p.nseg) {
+    if (lane < p.dstate) p.state_out[(b * p.dim + c) * p.dstate + lane] = carry;
+  }
+}
+
+// How a call runs here, if it does (sw == 0: it does not, scan.hip has it).
+struct Plan {
+  int layout, sw, nseg;
+};
+
+// Which calls: unit strides along one axis, B and C in x's type (anything else keeps scan.hip's
+// packed B/C), and few enough channels.  Measured (us, fp16 unless said, dstate 16, scan.hip
+// against this):
+//   2 to 8 thousand channels: 4x2048x2048 (B x D x L) 125 -> 101 along time, 138 -> 114 along
+//     channels; 4x1536x8192 351 -> 293 and 404 -> 351; 1x2048x2048 48 -> 37 and 53 -> 45.  Above,
+//     scan.hip's chains fill the chip: 4x3072x2048 137 against 145 along time; by rows equal
+//     at 12 thousand (160, 164) and ahead at 10 (4x2560x2048 170 -> 141).  Steps padded to whole
+//     chunks count as work: 4x1536x300 31 against 36.
+//   dstate > 16, where scan.hip has only 64-channel blocks: 2x1536x2048 at 32 states 347 -> 90,
+//     4x3072x2048 469 -> 263, at 40 thousand channels 345 against 424.
+//   fewer: one chunk always (1x1536x512 22 -> 12).  Long sequences on 512 to 1536 channels
+//     keep scan.hip's split over time, whose two passes take fewer slots (1x1024x32768 247
+//     against 292 here), up to lengths where one unsplit pass wins: 1x1536x2048 37 -> 35 and 44 ->
+//     43, 1x1024x2048 29 -> 25 and 32 against 38.  fp32 pays twice for its exponentials there:
+//     1x1024x8192 132 -> 116 along time.
+//   a few hundred and less: both passes here are short (1x16x32768 fp32 109 -> 21, 1x64x8192 37
+//     -> 18); 1x256x32768 93 against 104.
+inline Plan plan(const mm_scan_params* a, size_t sum_bytes) {
+  Plan pl = {kTime, 0, 1};
+  const int64_t ch = a->batch * a->dim, L = a->seqlen;
+  if (L < 8 || L > (1 << 30) || ch > (1 << 20) || a->bc_dtype != a->x_dtype) return pl;
+  bool time_c = a->B_stride[2] == 1 && a->C_stride[2] == 1;
+  bool chan_c = a->B_stride[1] == 1 && a->C_stride[1] == 1 && a->dim % 8 == 0 && a->dstate % 8 == 0;
+  const int64_t* st[4] = {a->u_stride, a->delta_stride, a->y_stride, a->z_stride};
+  for (int i = 0; i < (a->z ? 4 : 3); ++i) {
+    time_c = time_c && st[i][2] == 1;
+    chan_c = chan_c && st[i][1] == 1;
+  }
+  if (!time_c && !chan_c) return pl;
+  pl.layout = time_c ? kTime : kRows;
+  const bool f32 = a->x_dtype == MM_F32;
+  const int64_t nch = ceil_div(L, kChunk);
+
+  const int64_t most = a->dstate > 16 ? 16384 : time_c || f32 ? 8192 : 10240;
+  if (ch * nch * kChunk > most * L) return pl;
+  bool split = false;
+  if (a->dstate > 16) {
+    split = ch <= 512 && nch > 2;
+  } else if (nch == 1) {
+  } else if (time_c) {
+    if (ch >= (f32 ? 1024 : 2048)) {
+    } else if (ch >= 512 && nch <= (ch >= 768 ? 4 : 2)) {
+    } else if ((ch <= 512 && ch * nch <= 2048) || (ch <= 256 && ch * nch <= 4096)) {
+      split = nch > 2;
+    } else {
+      return pl;
+    }
+  } else {
+    if (ch >= 3072 || (ch >= (f32 ? 1024 : 2048) && nch <= 8)) {
+    } else if (ch >= 1536 && nch <= 4) {
+    } else if (ch >= 768 && nch <= 2) {
+    } else if (ch <= 256 && nch >= 4 && ch * nch <= 4096) {
+      split = true;
+    } else {
+      return pl;
+    }
+  }
+
+  // Waves per channel.  Unsplit, until the channels alone give four waves per SIMD: 1x1536x2048
+  // fp32 61 (SW = 1), 52 (2), 48 us (4), 2x1536x4096 fp16 104, 95, 114; by rows a second wave
+  // pays below 1536 channels, in fp32 below 2048.  Split, as long as the segments leave room.
+  const int64_t seg = std::min<int64_t>(nch, kMaxSeg);
+  if (split) {
+    const int64_t bytes = 4 * ch * (a->dstate + 1);
+    int64_t nseg = std::min<int64_t>({seg, static_cast<int64_t>(sum_bytes) / bytes, std::max<int64_t>(1, 4096 / ch)});
+    if (nseg > 1) {
+      const int64_t per = ceil_div(nch, nseg);
+      pl.nseg = static_cast<int>(ceil_div(nch, per));
+    }
+    const int64_t w = ch * pl.nseg;
+    pl.sw = time_c ? (w <= 1024 ? 4 : w <= 2048 ? 2 : 1) : (w <= 2048 ? 2 : 1);
+  } else {
+    pl.sw = time_c ? (ch <= 1536 ? 4 : ch < 4096 ? 2 : 1) : (ch < (f32 ? 2049 : 1536) ? 2 : 1);
+  }
+  return pl;
+}
+
+bool preferred(const mm_scan_params* a, size_t sum_bytes) { return plan(a, sum_bytes).sw > 0; }
+
+template <int DT, int LAYOUT, int CH, int SW>
+void launch_n(const Params& p, int64_t batch, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(ceil_div(p.dim, CH) * p.nseg * batch));
+  const dim3 block(64 * CH * SW);
+  if (p.nseg > 1)
+    hipLaunchKernelGGL((lane_scan_kernel<DT, LAYOUT, true, CH, SW>), grid, block, 0, s, p);
+  hipLaunchKernelGGL((lane_scan_kernel<DT, LAYOUT, false, CH, SW>), grid, block, 0, s, p);
+}
+
+template <int DT>
+void launch_dt(const Params& p, int64_t batch, const Plan& pl, hipStream_t s) {
+  if (pl.layout == kTime) {
+    if (pl.sw == 4) launch_n<DT, kTime, 2, 4>(p, batch, s);
+    else if (pl.sw == 2) launch_n<DT, kTime, 4, 2>(p, batch, s);
+    else launch_n<DT, kTime, 8, 1>(p, batch, s);
+  } else {
+    if (pl.sw == 2) launch_n<DT, kRows, 8, 2>(p, batch, s);
+    else launch_n<DT, kRows, 8, 1>(p, batch, s);
+  }
+}
+
+int launch(const mm_scan_params* a, int* ctl, float* sum, size_t sum_bytes, void* stream) {
+  const Plan pl = plan(a, sum_bytes);
+  Params p = {};
+  p.u = a->u;
+  p.delta = a->delta;
+  p.z = a->z;
+  p.y = a->y;
+  p.A = a->A;
+  p.D = a->D;
+  p.B = a->B;
+  p.C = a->C;
+  p.state_out = a->state_out;
+  p.sum = sum;
+  p.ctl = ctl;
+  p.us0 = a->u_stride[0], p.us1 = a->u_stride[1], p.us2 = a->u_stride[2];
+  p.ds0 = a->delta_stride[0], p.ds1 = a->delta_stride[1], p.ds2 = a->delta_stride[2];
+  p.zs0 = a->z_stride[0], p.zs1 = a->z_stride[1], p.zs2 = a->z_stride[2];
+  p.ys0 = a->y_stride[0], p.ys1 = a->y_stride[1], p.ys2 = a->y_stride[2];
+  p.Bs0 = a->B_stride[0], p.Bs1 = a->B_stride[1], p.Bs2 = a->B_stride[2];
+  p.Cs0 = a->C_stride[0], p.Cs1 = a->C_stride[1], p.Cs2 = a->C_stride[2];
+  p.As0 = a->A_stride[0], p.As1 = a->A_stride[1];
+  p.Ds = a->D_stride;
+  p.dim = static_cast<int32_t>(a->dim);
+  p.dstate = static_cast<int32_t>(a->dstate);
+  p.seqlen = static_cast<int32_t>(a->seqlen);
+  p.softplus_cut = a->delta_softplus ? 20.0f : __builtin_nanf("");
+  p.nseg = pl.nseg;
+  p.seg_chunks = static_cast<int32_t>(ceil_div(ceil_div(a->seqlen, kChunk), pl.nseg));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (a->x_dtype) {
+    case MM_F32: launch_dt<MM_F32>(p, a->batch, pl, s); break;
+    case MM_F16: launch_dt<MM_F16>(p, a->batch, pl, s); break;
+    default: launch_dt<MM_BF16>(p, a->batch, pl, s); break;
+  }
+  return check_launch("lane_scan");
+}
+
+}  // namespace lscan
+}  // namespace mm

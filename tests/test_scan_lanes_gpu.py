@@ -1,0 +1,92 @@
+"""The scan with time across the lanes (csrc/scan_lanes.hip): chunk, lane and state edges, each
+way of sharing the states among waves, time split into segments, growing states -- against the
+fp64 oracle at test_scan_gpu's bars, and against the general path on the same values."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_close, config0_inputs, features_inputs
+from test_scan_gpu import TOL, check, gpu_scan, oracle_scan
+
+pytestmark = pytest.mark.gpu
+
+# (batch, dim, dstate, seqlen): one vector of steps; ends inside a chunk, a lane and a vector; one
+# whole chunk; a few elements past one; several state groups, the last one partial
+EDGES = [(1, 8, 16, 8), (1, 1, 1, 9), (2, 13, 5, 511), (1, 24, 16, 512), (3, 40, 16, 513),
+         (1, 16, 24, 1025), (2, 8, 64, 700), (1, 7, 33, 1543)]
+# states shared by 4, 2 and 1 waves; two launches (segments), the first and last of one chunk or two
+SHAPES = EDGES + [(1, 1100, 16, 530), (1, 2048, 16, 601), (2, 2100, 16, 520), (1, 16, 16, 9001),
+                  (1, 256, 16, 2100), (1, 64, 16, 32769), (1, 512, 32, 1030)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_time_contiguous(oracle_lib, dev, shape, dtype):
+    check(oracle_lib, dev, config0_inputs(*shape, seed=sum(shape)), f"lanes {shape}", dtype=dtype, softplus=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s[1] % 8 == 0 and s[2] % 8 == 0], ids=str)
+def test_channel_contiguous(oracle_lib, dev, shape, dtype):
+    check(oracle_lib, dev, config0_inputs(*shape, seed=sum(shape)), f"lanes {shape}", dtype=dtype, softplus=True,
+          layout="bld")
+
+
+@pytest.mark.parametrize("use_D,use_z,softplus", [(False, False, False), (True, False, True), (False, True, False)])
+@pytest.mark.parametrize("layout", ["bdl", "bld"])
+def test_options(oracle_lib, dev, use_D, use_z, softplus, layout):
+    inp = features_inputs(2, 24, 16, 1100, seed=3)
+    if not softplus:
+        inp["delta"] = np.abs(inp["delta"]) * 0.1
+    check(oracle_lib, dev, inp, f"lanes D={use_D} z={use_z}", softplus=softplus, use_D=use_D, use_z=use_z, layout=layout)
+
+
+def _general_path(inp, dev, dtype):
+    """The same values through scan.hip: tensors of no unit stride take its element-wise loads."""
+    return gpu_scan(inp, dev, dtype, softplus=True, layout="gather")
+
+
+@pytest.mark.parametrize("layout", ["bdl", "bld"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(2, 40, 16, 777), (1, 2048, 8, 300), (1, 32, 16, 5000)], ids=str)
+def test_matches_general_path(dev, shape, dtype, layout):
+    inp = config0_inputs(*shape, seed=4)
+    y, h = gpu_scan(inp, dev, dtype, softplus=True, layout=layout)
+    yg, hg = _general_path(inp, dev, dtype)
+    rt, at = TOL[dtype]
+    assert_close(y, yg, rt, at, "y")
+    assert_close(h, hg, 1e-5, 1e-5, "state")  # fp32 state either way
+
+
+@pytest.mark.parametrize("layout", ["bdl", "bld"])
+@pytest.mark.parametrize("shape,quiet", [((1, 16, 16, 600), 400), ((1, 16, 16, 2000), 1850)], ids=str)
+def test_growing_states(oracle_lib, dev, layout, shape, quiet):
+    """A > 0: the product of decays over a chunk overflows fp32 (exp(0.3 x 600) and more) while the
+    states, zero for the first `quiet` steps, stay finite (they grow for 200 steps at most)."""
+    inp = config0_inputs(*shape, seed=6)
+    inp["delta"][:] = 1.0
+    inp["A"] = np.broadcast_to(np.linspace(-0.5, 0.3, shape[2], dtype=np.float32), inp["A"].shape).copy()
+    inp["u"][..., :quiet] = 0.0
+    y, h = gpu_scan(inp, dev, layout=layout)
+    yo, ho = oracle_scan(oracle_lib, inp)
+    # |y| reaches e^60 (relative bar 1e-4: ~200 fp32 steps at 2^-24 each, growing with the state)
+    assert np.isfinite(y).all()
+    assert_close(y, yo, 1e-4, 1e-5 * np.abs(yo).max(axis=(0, 1)).clip(1.0), "y")
+    assert_close(h, ho, 1e-4, 1e-5 * np.abs(ho).max(), "state")
+
+
+def test_nan_stays_behind(dev):
+    """A NaN input reaches no earlier step and no other channel."""
+    inp = config0_inputs(1, 16, 16, 1500, seed=7)
+    ref, _ = gpu_scan(inp, dev, softplus=True)
+    inp["u"][0, 3, 700] = np.nan
+    for layout in ("bdl", "bld"):
+        y, _ = gpu_scan(inp, dev, softplus=True, layout=layout)
+        assert np.isnan(y[0, 3, 700:]).all()
+        keep = np.ones_like(y, bool)
+        keep[0, 3, 700:] = False
+        assert np.isfinite(y[keep]).all()
+        assert_close(y[keep], ref[keep], 1e-5, 1e-5, layout)
