@@ -6,10 +6,13 @@
 // fp16 vector when channels are contiguous) and a run of TC timesteps; the
 // (width-1)-deep causal window lives in registers and slides along time, so x
 // is read once (plus a (width-1)-step halo per run) and out written once:
-// HBM-bound at ~2 x element size bytes per (b, t, c).  The run is walked in groups
-// of kU steps whose loads are all issued before any of them is used (clamped to the
-// run's last step, so every load is in bounds and unconditional): one load in flight
-// per thread left the kernel latency-bound at a third of the HBM rate.
+// HBM-bound at ~2 x element size bytes per (b, t, c) where there are enough runs (64 x 512 x
+// 5120 fp16: 140 us, 4.8 TB/s).  The run is walked in groups of kU steps whose loads are
+// all issued before any of them is used, the next group's during this one's arithmetic
+// (clamped to the run's last step, so every load is in bounds and unconditional): one load
+// in flight per thread left the kernel latency-bound at a third of the HBM rate.  Short
+// sequences are bound by a thread's own instructions: 1 x 64 x 1536 fp16 8.4 -> 5.7 us, 1 x 2048 x
+// 1536 9.3 -> 7.4, fp32 14.7 -> 9.4 (scalar run indexes, the loads above, fp32 taps as vectors).
 //
 // The decode step replaces mamba_block.py:170-177: shift the (batch, dim, width)
 // window left in place, append x, dot with the taps, add bias, SiLU.
@@ -22,7 +25,7 @@ namespace mm {
 namespace conv {
 
 constexpr int kCV = 8;      // channels per thread
-constexpr int kU = 8;       // timesteps per load group
+constexpr int kU = 4;       // timesteps per load group
 constexpr int kMaxW = 8;    // largest width accepted
 constexpr int kBlock = 256;
 
@@ -32,10 +35,12 @@ struct Params {
   const void* bias;
   void* out;
   void* state;
-  int64_t batch, seqlen, dim, width, tc, nchunks, ncg;
+  int64_t batch, seqlen, dim, width, tc, ncg, nruns;
+  uint32_t nchunks, ncgb;  // runs of a sequence; blocks of 64 channel groups
   int64_t xs0, xs1, xs2, os0, os1, os2, ws0, ws1;
   int32_t w_dtype, apply_silu, vec_ok;
-  int32_t w_vec;  // 2-byte taps in contiguous rows of 4 (and bias) on 16-byte boundaries
+  int32_t uni;    // a wave's lanes share one run
+  int32_t w_vec;  // taps in contiguous rows of 4, taps and bias aligned for vectors of 8
 };
 
 __device__ __forceinline__ float ld_any(const void* p, int64_t i, int32_t dt) {
@@ -44,19 +49,51 @@ __device__ __forceinline__ float ld_any(const void* p, int64_t i, int32_t dt) {
 
 // K = compile-time width; K == 0 means "runtime width <= kMaxW" using a zero-padded
 // kMaxW-tap window (taps aligned to the newest input).
-template <int DT, int K, bool VEC>
+template <int DT, int K, bool VEC, bool UNI>
 __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
   using T = typename Ty<DT>::T;
   using V8 = typename Ty<DT>::V8;
   constexpr int W = K > 0 ? K : kMaxW;
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  const int64_t total = p.batch * p.nchunks * p.ncg;
-  if (gid >= total) return;
-  const int64_t cg = gid % p.ncg;
-  const int64_t chunk = (gid / p.ncg) % p.nchunks;
-  const int64_t b = gid / (p.ncg * p.nchunks);
+  constexpr int U = VEC ? kU : 1;
+  // UNI: a wave is 64 neighbouring channel groups of one run, so the run's indexes are wave-uniform
+  // (scalar registers and arithmetic: with a run per thread their divisions and products were
+  // a third of a short run's instructions).  Otherwise groups and runs are one flat range.
+  int64_t cg;
+  std::conditional_t<UNI, uint32_t, int64_t> run;
+  if constexpr (UNI) {
+    cg = static_cast<int64_t>(blockIdx.x % p.ncgb) * 64 + (threadIdx.x & 63);
+    run = blockIdx.x / p.ncgb * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  } else {
+    const int64_t gid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    cg = gid % p.ncg;
+    run = gid / p.ncg;
+  }
+  if (cg >= p.ncg || run >= p.nruns) return;
+  const int64_t b = run / p.nchunks, chunk = run % p.nchunks;
   const int64_t c0 = cg * kCV;
   const int off = W - static_cast<int>(K > 0 ? K : p.width);  // leading zero taps (K == 0)
+
+  const int64_t t_begin = chunk * p.tc;
+  const int64_t t_end = std::min<int64_t>(t_begin + p.tc, p.seqlen);
+
+  // Vector path: the run's causal history and its first U steps, raw, ahead of everything that
+  // waits, so that one round trip to memory covers them and the taps.
+  // All loads are in bounds: steps before the sequence read step 0, steps past the run its last.
+  const T* const xb = static_cast<const T*>(p.x) + b * p.xs0 + c0;
+  V8 hr[VEC && W > 1 ? W - 1 : 1], xr[VEC ? U : 1];
+  auto load_group = [&](int64_t t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      xr[u] = *reinterpret_cast<const V8*>(xb + (t0 + u < t_end ? t0 + u : t_end - 1) * p.xs1);
+  };
+  if constexpr (VEC) {
+#pragma unroll
+    for (int k = 0; k < W - 1; ++k) {
+      const int64_t t = t_begin - (W - 1) + k;
+      hr[k] = *reinterpret_cast<const V8*>(xb + (t >= 0 ? t : 0) * p.xs1);
+    }
+    load_group(t_begin);
+  }
 
   // Taps (zero-padded at the old end when K == 0) and bias ((dim,) contiguous, w_dtype).
   // Every load is unconditional, from a clamped in-bounds address, and masked afterwards:
@@ -78,9 +115,9 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
       bias[j] = ld<WDT>(p.bias != nullptr ? p.bias : p.w, p.bias != nullptr ? cc : 0);
     }
   };
-  // Width 4 with 2-byte taps in contiguous (dim, 4) rows (the model's conv1d.weight): the
-  // thread's 8 channels x 4 taps are 64 contiguous bytes, read as four 16-byte loads, and
-  // its 8 biases as one.
+  // Width 4 with taps in contiguous (dim, 4) rows (the model's conv1d.weight): the thread's 8
+  // channels x 4 taps are 32 contiguous elements, read as four vectors of 8, and its 8 biases
+  // as one.
   auto load_taps_vec = [&](auto wdt) __attribute__((always_inline)) {
     constexpr int WDT = decltype(wdt)::value;
     using WV = typename Ty<WDT>::V8;
@@ -100,7 +137,8 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
   bool taps_done = false;
   if constexpr (K == 4) {
     if (p.w_vec) {
-      if (p.w_dtype == MM_F16) load_taps_vec(std::integral_constant<int, MM_F16>{});
+      if (p.w_dtype == MM_F32) load_taps_vec(std::integral_constant<int, MM_F32>{});
+      else if (p.w_dtype == MM_F16) load_taps_vec(std::integral_constant<int, MM_F16>{});
       else load_taps_vec(std::integral_constant<int, MM_BF16>{});
       taps_done = true;
     }
@@ -118,56 +156,42 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
     bias[j] = (cin && p.bias != nullptr) ? bias[j] : 0.0f;
   }
 
-  // x[b, t, c0 .. c0 + 7] (t >= 0); channels past dim read as zero.
-  // Unconditional loads here too: on the vector path every thread's channel group lies
-  // inside dim (dim % 8 == 0); the strided path reads channel 0 past dim and masks.
+  // Strided path: x[b, t, c0 .. c0 + 7] (t >= 0) element by element; channels past dim read
+  // channel 0 and count as zero.
   auto load_x = [&](int64_t t, float v[kCV]) {
     const T* xp = static_cast<const T*>(p.x) + b * p.xs0 + t * p.xs1;
-    if constexpr (VEC) {
-      const V8 r = *reinterpret_cast<const V8*>(xp + c0);
+    float raw[kCV];
 #pragma unroll
-      for (int j = 0; j < kCV; ++j) v[j] = Ty<DT>::f(r[j]);
-    } else {
-      float raw[kCV];
+    for (int j = 0; j < kCV; ++j) raw[j] = Ty<DT>::f(xp[(c0 + j < p.dim ? c0 + j : 0) * p.xs2]);
 #pragma unroll
-      for (int j = 0; j < kCV; ++j) raw[j] = Ty<DT>::f(xp[(c0 + j < p.dim ? c0 + j : 0) * p.xs2]);
-#pragma unroll
-      for (int j = 0; j < kCV; ++j) v[j] = (c0 + j < p.dim) ? raw[j] : 0.0f;
-    }
+    for (int j = 0; j < kCV; ++j) v[j] = (c0 + j < p.dim) ? raw[j] : 0.0f;
   };
 
-  const int64_t t_begin = chunk * p.tc;
-  const int64_t t_end = std::min<int64_t>(t_begin + p.tc, p.seqlen);
-
-  // win[k] holds x[t - (W-1) + k] for k < W-1 (the causal history): loaded from step 0
-  // where t < 0 (unconditional loads, see the taps) and zeroed after.
+  // win[k] holds x[t - (W-1) + k] for k < W-1 (the causal history): zero where t < 0.
   float win[W > 1 ? W - 1 : 1][kCV];
 #pragma unroll
   for (int k = 0; k < W - 1; ++k) {
     const int64_t t = t_begin - (W - 1) + k;
-    load_x(t >= 0 ? t : 0, win[k]);
-  }
+    if constexpr (VEC) {
 #pragma unroll
-  for (int k = 0; k < W - 1; ++k) {
-    const bool tin = t_begin - (W - 1) + k >= 0;
+      for (int j = 0; j < kCV; ++j) win[k][j] = Ty<DT>::f(hr[k][j]);
+    } else {
+      load_x(t >= 0 ? t : 0, win[k]);
+    }
 #pragma unroll
-    for (int j = 0; j < kCV; ++j) win[k][j] = tin ? win[k][j] : 0.0f;
+    for (int j = 0; j < kCV; ++j) win[k][j] = t >= 0 ? win[k][j] : 0.0f;
   }
 
-  // Vector path: the group's raw 16-byte rows are loaded before any is converted (every
-  // thread's channel group is inside dim there, so no load is guarded).
-  constexpr int U = VEC ? kU : 1;
-  const T* const xb = static_cast<const T*>(p.x) + b * p.xs0 + c0;
   for (int64_t t0 = t_begin; t0 < t_end; t0 += U) {
-  V8 xr[U];
-  float xs[VEC ? 1 : kCV];
-  if constexpr (VEC) {
+    V8 cur[VEC ? U : 1];
+    float xs[kCV];
+    if constexpr (VEC) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      xr[u] = *reinterpret_cast<const V8*>(xb + (t0 + u < t_end ? t0 + u : t_end - 1) * p.xs1);
-  } else {
-    load_x(t0, xs);
-  }
+      for (int u = 0; u < U; ++u) cur[u] = xr[u];
+      if (t0 + U < t_end) load_group(t0 + U);  // in flight during this group's arithmetic
+    } else {
+      load_x(t0, xs);
+    }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t t = t0 + u;
@@ -175,7 +199,7 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
     float xn[kCV];
 #pragma unroll
     for (int j = 0; j < kCV; ++j) {
-      if constexpr (VEC) xn[j] = Ty<DT>::f(xr[u][j]);
+      if constexpr (VEC) xn[j] = Ty<DT>::f(cur[u][j]);
       else xn[j] = xs[j];
     }
     float o[kCV];
@@ -189,12 +213,10 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
     }
     T* op = static_cast<T*>(p.out) + b * p.os0 + t * p.os1;
     if constexpr (VEC) {
-      if (c0 < p.dim) {
-        V8 r;
+      V8 r;
 #pragma unroll
-        for (int j = 0; j < kCV; ++j) r[j] = Ty<DT>::from(o[j]);
-        *reinterpret_cast<V8*>(op + c0) = r;
-      }
+      for (int j = 0; j < kCV; ++j) r[j] = Ty<DT>::from(o[j]);
+      *reinterpret_cast<V8*>(op + c0) = r;
     } else {
 #pragma unroll
       for (int j = 0; j < kCV; ++j)
@@ -231,19 +253,22 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
 
 template <int DT>
 void launch_dt(const Params& p, hipStream_t s) {
-  const int64_t total = p.batch * p.nchunks * p.ncg;
-  const dim3 grid(static_cast<unsigned>(ceil_div(total, kBlock)));
-#define MM_CONV_W(V)                                                                          \
+  const int64_t blocks =
+      p.uni ? p.ncgb * ceil_div(p.nruns, kBlock / 64) : ceil_div(p.nruns * p.ncg, kBlock);
+  const dim3 grid(static_cast<unsigned>(blocks));
+#define MM_CONV_W(V, U)                                                                         \
   switch (p.width) {                                                                          \
-    case 2: hipLaunchKernelGGL((conv1d_kernel<DT, 2, V>), grid, dim3(kBlock), 0, s, p); break; \
-    case 3: hipLaunchKernelGGL((conv1d_kernel<DT, 3, V>), grid, dim3(kBlock), 0, s, p); break; \
-    case 4: hipLaunchKernelGGL((conv1d_kernel<DT, 4, V>), grid, dim3(kBlock), 0, s, p); break; \
-    default: hipLaunchKernelGGL((conv1d_kernel<DT, 0, V>), grid, dim3(kBlock), 0, s, p); break; \
+    case 2: hipLaunchKernelGGL((conv1d_kernel<DT, 2, V, U>), grid, dim3(kBlock), 0, s, p); break; \
+    case 3: hipLaunchKernelGGL((conv1d_kernel<DT, 3, V, U>), grid, dim3(kBlock), 0, s, p); break; \
+    case 4: hipLaunchKernelGGL((conv1d_kernel<DT, 4, V, U>), grid, dim3(kBlock), 0, s, p); break; \
+    default: hipLaunchKernelGGL((conv1d_kernel<DT, 0, V, U>), grid, dim3(kBlock), 0, s, p); break; \
   }
-  if (p.vec_ok) {
-    MM_CONV_W(true)
+  if (p.uni) {
+    MM_CONV_W(true, true)
+  } else if (p.vec_ok) {
+    MM_CONV_W(true, false)
   } else {
-    MM_CONV_W(false)
+    MM_CONV_W(false, false)
   }
 #undef MM_CONV_W
 }
@@ -367,16 +392,28 @@ int mm_causal_conv1d_fwd(const void* x, const void* weight, const void* bias, vo
                  ? 1
                  : 0;
   p.ncg = ceil_div(dim, kCV);
-  p.w_vec = (width == 4 && w_dtype != MM_F32 && p.ws1 == 1 && p.ws0 == 4 && dim % kCV == 0 &&
-             aligned(weight, 16) && (bias == nullptr || aligned(bias, 16)))
+  p.ncgb = static_cast<uint32_t>(ceil_div(p.ncg, 64));
+  const int64_t wb = kCV * dtype_size(w_dtype);
+  p.w_vec = (width == 4 && p.ws1 == 1 && p.ws0 == 4 && dim % kCV == 0 && aligned(weight, wb) &&
+             (bias == nullptr || aligned(bias, wb)))
                 ? 1
                 : 0;
-  // Run length: enough runs for >= ~256k threads (~16 waves per CU), runs of at most
-  // 256 steps and at least kU (one load group; the (width-1)-step halo is re-read per run).
-  int64_t tc = 256;
-  while (tc > kU && batch * p.ncg * ceil_div(seqlen, tc) < 262144) tc /= 2;
+  // Whole waves on one run where that leaves at most an eighth of the lanes idle (4 x 2048 x 1800
+  // fp16 19.8 -> 16.6 us; 1544 channels, a quarter idle, 18.4 -> 20.6).
+  p.uni = p.vec_ok && 8 * p.ncg >= 7 * 64 * static_cast<int64_t>(p.ncgb);
+  // Run length: 32 steps, shorter while there are at most 65536 threads (one wave per SIMD)
+  // and down to one load group (the (width-1)-step history is re-read per run).  fp16, us at
+  // 4 / 8 / 16 / 32 steps: 2 x 1021 x 1024 5.2 / 6.3 / 8.9 / 13.6, 4 x 2048 x 1536 18.2 / 16.3 / 15.7
+  // / 16.4, 8 x 1024 x 2048 23.6 / 21.9 / 18.9 / 17.1, 64 x 512 x 5120 179 / 154 / 139 / 140.
+  // The flat range spends more per run and wants more waves, and runs of 8 at least: 4 x 2048 x 1032
+  // 14.9 us at 8 steps, 16.0 at 16; 3 x 777 x 1542 17.9 at 8, 22.0 at 4.
+  const int64_t least = p.uni ? kU : 2 * kU, few = p.uni ? 65536 : 131072;
+  int64_t tc = 32;
+  while (tc > least && batch * p.ncg * ceil_div(seqlen, tc) <= few) tc /= 2;
   p.tc = tc;
-  p.nchunks = ceil_div(seqlen, tc);
+  p.nchunks = static_cast<uint32_t>(ceil_div(seqlen, tc));
+  p.nruns = batch * ceil_div(seqlen, tc);
+  if (p.nruns * p.ncgb > 0x7fffffff) p.uni = 0;
 
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (x_dtype) {

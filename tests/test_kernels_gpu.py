@@ -275,3 +275,26 @@ def test_argmax_rows(dev, n, dtype):
     # strided rows (a column slice of a wider buffer)
     wide = torch.randn((9, n + 24), generator=g, device=dev).to(dtype)
     assert torch.equal(argmax_rows(wide[:, :n]), torch.argmax(wide[:, :n], dim=-1))
+
+
+# Runs of 4 to 32 steps with a history on every boundary, sequences that end inside a run and a load
+# group, channel groups that end inside a wave's 64, taps as vectors in each type.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,L,D", [(1, 1, 8), (1, 5, 520), (3, 66, 504), (2, 37, 4104), (1, 1030, 1536),
+                                   (5, 33, 16384), (2, 2047, 2056)])
+def test_causal_conv1d_runs(dev, B, L, D, dtype):
+    from mamba_metal_amd.conv1d import causal_conv1d
+
+    rng = np.random.default_rng(B + L + D)
+    r = lambda *s: torch.as_tensor(rng.standard_normal(s).astype(np.float32)).to(dtype)
+    x, w, b = r(B, L, D), r(D, 1, 4), r(D)
+    state = torch.empty((B, D, 4), dtype=dtype, device=dev)
+    y = causal_conv1d(x.to(dev), w.to(dev), b.to(dev), apply_silu=True, conv_state_out=state)
+    xd = torch.cat([torch.zeros(B, 3, D), x.float()], 1).double()
+    ref = sum(xd[:, k:k + L] * w.double()[:, 0, k] for k in range(4)) + b.double()
+    ref = torch.nn.functional.silu(ref)
+    # four fp32 fmas and SiLU on the hardware's exp and rcp (~1e-6), then the output's half ulp
+    tol = {torch.float32: 4e-6, torch.float16: 2.0 ** -11 + 4e-6, torch.bfloat16: 2.0 ** -8}[dtype]
+    assert_close(y.float().cpu().numpy(), ref.numpy(), tol, 4e-6, "conv")
+    last = torch.cat([torch.zeros(B, 4, D, dtype=dtype), x], 1)[:, -4:].transpose(1, 2)
+    assert torch.equal(state.cpu(), last), "conv state"
