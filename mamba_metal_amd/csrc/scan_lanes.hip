@@ -621,8 +621,12 @@ inline Plan plan(const mm_scan_params* a, size_t sum_bytes) {
   }
 
   // Waves per channel.  Unsplit, until the channels alone give four waves per SIMD: 1x1536x2048
-  // fp32 61 (SW = 1), 52 (2), 48 us (4), 2x1536x4096 fp16 104, 95, 114; by rows a second wave
-  // pays below 1536 channels, in fp32 below 2048.  Split, as long as the segments leave room.
+  // fp32 61 (SW = 1), 52 (2), 48 us (4), 2x1536x4096 fp16 104, 95, 114; by rows a second wave,
+  // on four channels a workgroup instead of eight, pays below 1536 channels and in fp32 always (B x
+  // L x D, against eight channels on one wave each): fp16 1x1000x1024 20.7 -> 15.2, 2x700x512 19.9
+  // -> 14.3, 1x2048x1536 40.8 and 41.2, 4x2048x1536 88 and 107; fp32 1x2048x1536 71 -> 55,
+  // 1x2048x3072 108 -> 82, 4x2048x1536 165 -> 147 (two waves on eight channels: 20.7, 19.5, 42.6,
+  // 121; 57, 109, 166).  Split, as long as the segments leave room.
   const int64_t seg = std::min<int64_t>(nch, kMaxSeg);
   if (split) {
     const int64_t bytes = 4 * ch * (a->dstate + 1);
@@ -634,7 +638,7 @@ inline Plan plan(const mm_scan_params* a, size_t sum_bytes) {
     const int64_t w = ch * pl.nseg;
     pl.sw = time_c ? (w <= 1024 ? 4 : w <= 2048 ? 2 : 1) : (w <= 2048 ? 2 : 1);
   } else {
-    pl.sw = time_c ? (ch <= 1536 ? 4 : ch < 4096 ? 2 : 1) : (ch < (f32 ? 2049 : 1536) ? 2 : 1);
+    pl.sw = time_c ? (ch <= 1536 ? 4 : ch < 4096 ? 2 : 1) : (f32 || ch < 1536 ? 2 : 1);
   }
   return pl;
 }
@@ -657,7 +661,7 @@ void launch_dt(const Params& p, int64_t batch, const Plan& pl, hipStream_t s) {
     else if (pl.sw == 2) launch_n<DT, kTime, 4, 2>(p, batch, s);
     else launch_n<DT, kTime, 8, 1>(p, batch, s);
   } else {
-    if (pl.sw == 2) launch_n<DT, kRows, 8, 2>(p, batch, s);
+    if (pl.sw == 2) launch_n<DT, kRows, 4, 2>(p, batch, s);
     else launch_n<DT, kRows, 8, 1>(p, batch, s);
   }
 }

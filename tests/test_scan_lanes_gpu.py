@@ -35,6 +35,15 @@ def test_channel_contiguous(oracle_lib, dev, shape, dtype):
           layout="bld")
 
 
+@pytest.mark.parametrize("shape", [(1, 1528, 16, 520), (1, 1536, 16, 520), (1, 2056, 8, 513), (3, 1000, 24, 40)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_channel_contiguous_wave_counts(oracle_lib, dev, shape, dtype):
+    """Either side of the channel count up to which two waves share a channel of 16-bit rows, more
+    channels in fp32 (two waves always), and channel groups of four with one, two and three state groups."""
+    check(oracle_lib, dev, config0_inputs(*shape, seed=sum(shape)), f"lanes {shape}", dtype=dtype, softplus=True,
+          layout="bld")
+
+
 @pytest.mark.parametrize("use_D,use_z,softplus", [(False, False, False), (True, False, True), (False, True, False)])
 @pytest.mark.parametrize("layout", ["bdl", "bld"])
 def test_options(oracle_lib, dev, use_D, use_z, softplus, layout):
