@@ -20,7 +20,8 @@
 // per update, 98% of the VALU's cycles busy), against 9.6-12 slots for scan.hip where that one's
 // chains fill the chip, and its 14-40 where they do not.  Tried and not kept: 16 steps per
 // lane (11 slots, but two waves per SIMD instead of four: B=4 D=1536 L=4096 149 -> 180 us), two
-// states interleaved per wave (149 -> 186), the next state's LDS reads ahead (149 -> 151).
+// states interleaved per wave where the chip is full (149 -> 186), the next state's LDS reads ahead
+// (149 -> 151), by rows both state groups of B and C loaded together (1x2048x1536 40.8 -> 42.8).
 #include <algorithm>
 #include <type_traits>
 
@@ -131,6 +132,37 @@ __device__ __forceinline__ void lane_scan(float& P, float& h, float pr, float ph
       : "v"(pr), "v"(ph));
 }
 
+// lane_scan of two states: the second's instructions stand where the first's results would be waited
+// for, so fewer s_nops are left.
+__device__ __forceinline__ void lane_scan2(float& P0, float& h0, float pr0, float ph0, float& P1, float& h1,
+                                           float pr1, float ph1) {
+  asm volatile(
+      "s_nop 1\n\t"
+      "v_fmac_f32_dpp %1, %1, %0 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_fmac_f32_dpp %3, %3, %2 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %2, %2, %2 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_fmac_f32_dpp %1, %1, %0 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_fmac_f32_dpp %3, %3, %2 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %2, %2, %2 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_fmac_f32_dpp %1, %1, %0 row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_fmac_f32_dpp %3, %3, %2 row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_mul_f32_dpp %2, %2, %2 row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_fmac_f32_dpp %1, %1, %0 row_shr:8 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_fmac_f32_dpp %3, %3, %2 row_shr:8 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "s_nop 0\n\t"
+      "v_fmac_f32_dpp %1, %1, %4 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %3, %3, %6 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+      "s_nop 0\n\t"
+      "v_fmac_f32_dpp %1, %1, %5 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %3, %3, %7 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+      "s_nop 1"
+      : "+&v"(P0), "+&v"(h0), "+&v"(P1), "+&v"(h1)
+      : "v"(pr0), "v"(ph0), "v"(pr1), "v"(ph1));
+}
+
 // B and C of NG states of a chunk on their way to LDS rows of fp32, zero past the sequence's
 // end and past the last state: one vector of 8 steps of a state (kTime) or of 8 states of a
 // step (kRows) per thread and tensor.
@@ -229,10 +261,14 @@ struct Stage {
 
 // CH channels per workgroup, each on SW waves that share its states.  kDirect: a lane loads and
 // stores its own steps; otherwise every thread owns 8 / SW elements of the chunk (steps of a
-// channel, or channels of a step) and they pass through an LDS tile.
-template <int DT, int LAYOUT, bool SUM, int CH, int SW>
-__global__ __launch_bounds__(64 * CH * SW, 4) void lane_scan_kernel(const Params p) {
+// channel, or channels of a step) and they pass through an LDS tile.  PAIR: two states side by side, for
+// launches of at most one workgroup per CU (two waves per SIMD), where a state's dependent steps are
+// waited for; with more waves the second state's registers cost more than that (4x2048x1536 fp16 by
+// rows 88 -> 108 us).
+template <int DT, int LAYOUT, bool SUM, int CH, int SW, bool PAIR>
+__global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(const Params p) {
   using T = typename Ty<DT>::T;
+  static_assert(!(SUM && PAIR), "pairs for the pass that writes y");
   constexpr int NT = 64 * CH * SW;
   constexpr bool kDirect = LAYOUT == kTime && SW == 1;
   static_assert(LAYOUT == kTime || NT % kChunk == 0, "threads in whole chunks");
@@ -452,8 +488,59 @@ __global__ __launch_bounds__(64 * CH * SW, 4) void lane_scan_kernel(const Params
       }
 
       const int n_end = std::min((part + 1) * kStates, p.dstate - g0);
+      int n = part * kStates;
+      if constexpr (PAIR) {
+        if (!serial) {
 #pragma unroll 1
-      for (int n = part * kStates; n < n_end; ++n) {
+          for (; n + 2 <= n_end; n += 2) {
+            float cin[2], a[2][kTL], bb[2][kTL], h[2], P[2], Pr[2], Ph[2], hx[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const float A = lane_value(Al, g0 + n + i);
+              cin[i] = lane_value(carry, g0 + n + i);
+#pragma unroll
+              for (int q = 0; q < kTL / 4; ++q) {
+                const float4 v = *reinterpret_cast<const float4*>(&s_b[n + i][lds_lane(lane, q)]);
+                bb[i][4 * q] = du[4 * q] * v.x;
+                bb[i][4 * q + 1] = du[4 * q + 1] * v.y;
+                bb[i][4 * q + 2] = du[4 * q + 2] * v.z;
+                bb[i][4 * q + 3] = du[4 * q + 3] * v.w;
+              }
+#pragma unroll
+              for (int j = 0; j < kTL; ++j) a[i][j] = exp2_decay<DT>(d2[j] * A);
+              h[i] = lane == 0 ? cin[i] : 0.0f;
+              P[i] = exp2_decay<DT>(S * A);
+              Pr[i] = exp2_decay<DT>(Srow * A);
+              Ph[i] = exp2_decay<DT>(Shalf * A);
+            }
+#pragma unroll
+            for (int j = 0; j < kTL; ++j)
+#pragma unroll
+              for (int i = 0; i < 2; ++i) h[i] = __builtin_fmaf(a[i][j], h[i], bb[i][j]);
+            lane_scan2(P[0], h[0], Pr[0], Ph[0], P[1], h[1], Pr[1], Ph[1]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              hx[i] = dpp_or<kWaveShr1>(cin[i], h[i]);
+              carry = lane == g0 + n + i ? lane_value(h[i], 63) : carry;
+            }
+#pragma unroll
+            for (int q = 0; q < kTL / 4; ++q) {
+              const float4 v0 = *reinterpret_cast<const float4*>(&s_c[n][lds_lane(lane, q)]);
+              const float4 v1 = *reinterpret_cast<const float4*>(&s_c[n + 1][lds_lane(lane, q)]);
+              const float cc[2][4] = {{v0.x, v0.y, v0.z, v0.w}, {v1.x, v1.y, v1.z, v1.w}};
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                  hx[i] = __builtin_fmaf(a[i][4 * q + j], hx[i], bb[i][4 * q + j]);
+                  y[4 * q + j] = __builtin_fmaf(hx[i], cc[i][j], y[4 * q + j]);
+                }
+            }
+          }
+        }
+      }
+#pragma unroll 1
+      for (; n < n_end; ++n) {
         const float A = lane_value(Al, g0 + n), cin = lane_value(carry, g0 + n);
         float a[kTL], bb[kTL];
 #pragma unroll
@@ -622,8 +709,8 @@ inline Plan plan(const mm_scan_params* a, size_t sum_bytes) {
 
   // Waves per channel.  Unsplit, until the channels alone give four waves per SIMD: 1x1536x2048
   // fp32 61 (SW = 1), 52 (2), 48 us (4), 2x1536x4096 fp16 104, 95, 114; by rows a second wave,
-  // on four channels a workgroup instead of eight, pays below 1536 channels and in fp32 always (B x
-  // L x D, against eight channels on one wave each): fp16 1x1000x1024 20.7 -> 15.2, 2x700x512 19.9
+  // on four channels a workgroup instead of eight, pays up to 1024 channels (a workgroup per CU) and
+  // in fp32 always (B x L x D, against eight channels on one wave each): fp16 1x1000x1024 20.7 -> 15.2, 2x700x512 19.9
   // -> 14.3, 1x2048x1536 40.8 and 41.2, 4x2048x1536 88 and 107; fp32 1x2048x1536 71 -> 55,
   // 1x2048x3072 108 -> 82, 4x2048x1536 165 -> 147 (two waves on eight channels: 20.7, 19.5, 42.6,
   // 121; 57, 109, 166).  Split, as long as the segments leave room.
@@ -638,20 +725,20 @@ inline Plan plan(const mm_scan_params* a, size_t sum_bytes) {
     const int64_t w = ch * pl.nseg;
     pl.sw = time_c ? (w <= 1024 ? 4 : w <= 2048 ? 2 : 1) : (w <= 2048 ? 2 : 1);
   } else {
-    pl.sw = time_c ? (ch <= 1536 ? 4 : ch < 4096 ? 2 : 1) : (f32 || ch < 1536 ? 2 : 1);
+    pl.sw = time_c ? (ch <= 1536 ? 4 : ch < 4096 ? 2 : 1) : (f32 || ch <= 1024 ? 2 : 1);
   }
   return pl;
 }
 
 bool preferred(const mm_scan_params* a, size_t sum_bytes) { return plan(a, sum_bytes).sw > 0; }
 
-template <int DT, int LAYOUT, int CH, int SW>
+template <int DT, int LAYOUT, int CH, int SW, bool PAIR = false>
 void launch_n(const Params& p, int64_t batch, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(ceil_div(p.dim, CH) * p.nseg * batch));
   const dim3 block(64 * CH * SW);
   if (p.nseg > 1)
-    hipLaunchKernelGGL((lane_scan_kernel<DT, LAYOUT, true, CH, SW>), grid, block, 0, s, p);
-  hipLaunchKernelGGL((lane_scan_kernel<DT, LAYOUT, false, CH, SW>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((lane_scan_kernel<DT, LAYOUT, true, CH, SW, false>), grid, block, 0, s, p);
+  hipLaunchKernelGGL((lane_scan_kernel<DT, LAYOUT, false, CH, SW, PAIR>), grid, block, 0, s, p);
 }
 
 template <int DT>
@@ -661,6 +748,15 @@ void launch_dt(const Params& p, int64_t batch, const Plan& pl, hipStream_t s) {
     else if (pl.sw == 2) launch_n<DT, kTime, 4, 2>(p, batch, s);
     else launch_n<DT, kTime, 8, 1>(p, batch, s);
   } else {
+    // 16-bit, unsplit, at most a workgroup per CU: states in pairs (fp32's longer decays keep a SIMD's
+    // two waves busy: 1x1000x1024 19.7 and 19.6 us, 2x2048x3072 155 and 203)
+    if constexpr (DT != MM_F32) {
+      if (p.nseg == 1 && ceil_div(p.dim, pl.sw == 2 ? 4 : 8) * batch <= 256) {
+        if (pl.sw == 2) launch_n<DT, kRows, 4, 2, true>(p, batch, s);
+        else launch_n<DT, kRows, 8, 1, true>(p, batch, s);
+        return;
+      }
+    }
     if (pl.sw == 2) launch_n<DT, kRows, 4, 2>(p, batch, s);
     else launch_n<DT, kRows, 8, 1>(p, batch, s);
   }

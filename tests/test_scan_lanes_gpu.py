@@ -35,13 +35,23 @@ def test_channel_contiguous(oracle_lib, dev, shape, dtype):
           layout="bld")
 
 
-@pytest.mark.parametrize("shape", [(1, 1528, 16, 520), (1, 1536, 16, 520), (1, 2056, 8, 513), (3, 1000, 24, 40)], ids=str)
+@pytest.mark.parametrize("shape", [(1, 1024, 16, 520), (1, 1032, 16, 520), (1, 2056, 8, 513), (3, 1000, 24, 40)], ids=str)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_channel_contiguous_wave_counts(oracle_lib, dev, shape, dtype):
-    """Either side of the channel count up to which two waves share a channel of 16-bit rows, more
-    channels in fp32 (two waves always), and channel groups of four with one, two and three state groups."""
+    """Either side of the channel counts up to which two waves share a channel of 16-bit rows (1024) and
+    its states go in pairs (2048), more channels in fp32 (two waves always), one to three state groups."""
     check(oracle_lib, dev, config0_inputs(*shape, seed=sum(shape)), f"lanes {shape}", dtype=dtype, softplus=True,
           layout="bld")
+
+
+@pytest.mark.parametrize("shape", [(1, 16, 16, 700), (1, 1032, 16, 700)], ids=str)
+def test_channel_contiguous_slow_growth(oracle_lib, dev, shape):
+    """A > 0 in 16 bits: chunks whose decays may not be multiplied up leave the pairs (states grow by
+    e^(0.01 x 70) at most)."""
+    inp = config0_inputs(*shape, seed=8)
+    inp["delta"][:] = 0.1
+    inp["A"] = np.broadcast_to(np.linspace(-20.0, 0.01, shape[2], dtype=np.float32), inp["A"].shape).copy()
+    check(oracle_lib, dev, inp, f"lanes growth {shape}", dtype=torch.float16, layout="bld")
 
 
 @pytest.mark.parametrize("use_D,use_z,softplus", [(False, False, False), (True, False, True), (False, True, False)])
