@@ -235,18 +235,26 @@ struct Stage {
             *reinterpret_cast<float4*>(&dst[n][lds_pos(t + q)]) = make_float4(
                 Ty<DT>::f(v[x][q]), Ty<DT>::f(v[x][q + 1]), Ty<DT>::f(v[x][q + 2]), Ty<DT>::f(v[x][q + 3]));
         } else {
-          // elements go to their own steps (the clamped vector's first ones once more, with the
-          // same values); steps past the end are zeroed.  tt is opaque: these positions are not
-          // worth registers in every chunk.
-          const bool nin = g0 + n < p.dstate;
-          int tt = t;
-          asm volatile("" : "+v"(tt));
-          const int back = std::max(t0 + tt - (p.seqlen - 8), 0);
+          // Vectors past the end and past the last state as zeros.  The one that holds the end was read
+          // 8 steps before it: its elements are moved down to their own steps through LDS, by eight
+          // lanes of its wave (which has this state alone, and whose LDS accesses stay in order), not
+          // in registers: code that runs once a call costs its fetches, 1x8x64 fp16 11 -> 7 us.
+          const bool in = g0 + n < p.dstate && t0 + t < p.seqlen;
 #pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            if (t0 + tt < p.seqlen && tt - back + k >= 0)
-              dst[n][lds_pos(tt - back + k)] = nin ? Ty<DT>::f(v[x][k]) : 0.0f;
-            if (t0 + tt + k >= p.seqlen) dst[n][lds_pos(tt + k)] = 0.0f;
+          for (int q = 0; q < 8; q += 4)
+            *reinterpret_cast<float4*>(&dst[n][lds_pos(t + q)]) =
+                make_float4(in ? Ty<DT>::f(v[x][q]) : 0.0f, in ? Ty<DT>::f(v[x][q + 1]) : 0.0f,
+                            in ? Ty<DT>::f(v[x][q + 2]) : 0.0f, in ? Ty<DT>::f(v[x][q + 3]) : 0.0f);
+          const int over = p.seqlen & 7, end = p.seqlen - over - t0;  // its steps inside, its first one
+          if (end < kChunk && over > 0) {
+            int l = item(tid) % kPer;
+            asm volatile("" : "+v"(l));  // not worth registers in every chunk
+            if (l < 8) {
+              asm volatile("" ::: "memory");  // the read is of another lane's store
+              const float f = dst[n][lds_pos(end + ((l - over) & 7))];
+              asm volatile("" ::: "memory");
+              dst[n][lds_pos(end + l)] = l < over ? f : 0.0f;
+            }
           }
         }
       } else {
@@ -379,8 +387,20 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
       if (t0 + kChunk <= p.seqlen) {
         v = *reinterpret_cast<const U*>(r);
       } else {
+        // The lane that holds the sequence's end reads its last E steps and moves them down to its
+        // own; lanes past it read step 0 (masked, see `inside`).
+        int left = p.seqlen - t0 - et;
+        asm volatile("" : "+v"(left));  // not worth registers in every chunk
+        const int off = left >= E ? et + t0 : left > 0 ? p.seqlen - E : 0;
+        v = *reinterpret_cast<const U*>(base + c * s1 + off);
+        if (left > 0 && left < E) {
 #pragma unroll
-        for (int k = 0; k < E; ++k) v[k] = t0 + et + k < p.seqlen ? r[k] : Ty<DT>::from(0.0f);
+          for (int m = 1; m < E; m *= 2) {
+            const bool by = (E - left) & m;
+#pragma unroll
+            for (int k = 0; k + m < E; ++k) v[k] = by ? v[k + m] : v[k];
+          }
+        }
       }
     } else {
       v = *reinterpret_cast<const U*>(base + (t0 + et < p.seqlen ? t0 + et : 0) * s2 + ch0 + ec);
@@ -622,7 +642,7 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
     if constexpr (LAYOUT == kTime) {
       T* const r = yp + c * p.ys1 + t0 + et;
       if (!chok) continue;
-      if (t0 + kChunk <= p.seqlen) {
+      if (t0 + et + E <= p.seqlen) {
         *reinterpret_cast<U*>(r) = o;
       } else {
 #pragma unroll

@@ -35,6 +35,16 @@ def test_channel_contiguous(oracle_lib, dev, shape, dtype):
           layout="bld")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim,first", [(8, 9), (1800, 513), (4104, 505)], ids=str)
+def test_every_end_of_a_vector(oracle_lib, dev, dim, first, dtype):
+    """Sequences that end after 1 .. 7 steps of a vector of 8, in one wave per channel and in two and
+    four: the vector with the end in it is read 8 (or a lane's) steps before the end and moved."""
+    for L in range(first, first + 7):
+        check(oracle_lib, dev, config0_inputs(1, dim, 16 if L % 2 else 5, L, seed=L), f"end {dim} {L}", dtype=dtype,
+              softplus=True)
+
+
 @pytest.mark.parametrize("shape", [(1, 1024, 16, 520), (1, 1032, 16, 520), (1, 2056, 8, 513), (3, 1000, 24, 40)], ids=str)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_channel_contiguous_wave_counts(oracle_lib, dev, shape, dtype):
