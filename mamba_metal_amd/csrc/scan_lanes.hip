@@ -83,6 +83,8 @@ constexpr int kWaveShr1 = 0x138; // lane i takes lane i - 1
 constexpr int kBcast15 = 0x142;  // rows 1 and 3 take the last lane of the row before
 constexpr int kBcast31 = 0x143;  // rows 2 and 3 take lane 31
 
+__device__ __forceinline__ bool is_inf(float v) { return __builtin_amdgcn_classf(v, 0x204); }
+
 __device__ __forceinline__ float lane_value(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
@@ -344,15 +346,15 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
         const int n = g0 + part * kStates + k;
         const float An = lane_value(Al, n & 63);
         float hin;
-        if (grows) {
+        if (grows || __any(is_inf(v[k]))) {
           hin = 0.0f;
           for (int i = seg - 1; i >= 0; --i) {
             // a segment's factor may overflow where its product with a small state does not: in
-            // sixteen steps (and not at all on a zero state)
+            // sixteen steps (and not at all on a zero or infinite state)
             const float f = exp2_decay<DT>(An * lane_value(ds, i) * 0.0625f);
             float g = hin;
             for (int r = 0; r < 16; ++r) g *= f;
-            hin = (hin == 0.0f ? 0.0f : g) + lane_value(v[k], i);
+            hin = (hin == 0.0f || is_inf(hin) ? hin : g) + lane_value(v[k], i);
           }
         } else {
           float vr, vh, va;
@@ -511,6 +513,12 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
       int n = part * kStates;
       if constexpr (PAIR) {
         if (!serial) {
+          float y_in[kTL];
+          const float carry_in = carry;
+          const int n_in = n;
+          float most = 0.0f;
+#pragma unroll
+          for (int j = 0; j < kTL; ++j) y_in[j] = y[j];
 #pragma unroll 1
           for (; n + 2 <= n_end; n += 2) {
             float cin[2], a[2][kTL], bb[2][kTL], h[2], P[2], Pr[2], Ph[2], hx[2];
@@ -537,6 +545,7 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
             for (int j = 0; j < kTL; ++j)
 #pragma unroll
               for (int i = 0; i < 2; ++i) h[i] = __builtin_fmaf(a[i][j], h[i], bb[i][j]);
+            most = fmaxf(fmaxf(most, fabsf(h[0])), fabsf(h[1]));
             lane_scan2(P[0], h[0], Pr[0], Ph[0], P[1], h[1], Pr[1], Ph[1]);
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
@@ -557,6 +566,12 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
                 }
             }
           }
+          if (__any(is_inf(most))) {  // the states once more below, see there
+            n = n_in;
+            carry = carry_in;
+#pragma unroll
+            for (int j = 0; j < kTL; ++j) y[j] = y_in[j];
+          }
         }
       }
 #pragma unroll 1
@@ -574,15 +589,23 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
 #pragma unroll
         for (int j = 0; j < kTL; ++j) a[j] = exp2_decay<DT>(d2[j] * A);
         float hx, hend;  // the state before this lane's steps, and at the chunk's end
+        bool one_by_one = serial;
         if (!serial) {
           float h = lane == 0 ? cin : 0.0f;
 #pragma unroll
           for (int j = 0; j < kTL; ++j) h = __builtin_fmaf(a[j], h, bb[j]);
+          // An infinite state stays infinite while each step's decay is above zero, but its product
+          // with the decay over many steps, which may underflow, is NaN: then, too, the lanes go
+          // one by one.  The test costs 0 to 4% of a call (1x1024x2048 fp16 21.7 -> 22.6 us, fp32 4x1024x4096
+          // 174 -> 175), one per chunk of its inputs or end states 1 to 12%; the pairs above test once
+          // a group of states and keep y as it was, for which the registers do not suffice here.
+          one_by_one = __any(is_inf(h));
           float P = exp2_decay<DT>(S * A);
           lane_scan(P, h, exp2_decay<DT>(Srow * A), exp2_decay<DT>(Shalf * A));
           hx = dpp_or<kWaveShr1>(cin, h);
           hend = lane_value(h, 63);
-        } else {
+        }
+        if (one_by_one) {
           hx = hend = cin;
           for (int l = 0; l < 64; ++l) {
             hx = lane == l ? hend : hx;

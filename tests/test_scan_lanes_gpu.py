@@ -119,3 +119,24 @@ def test_nan_stays_behind(dev):
         keep[0, 3, 700:] = False
         assert np.isfinite(y[keep]).all()
         assert_close(y[keep], ref[keep], 1e-5, 1e-5, layout)
+
+
+@pytest.mark.parametrize("layout", ["bdl", "bld"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 16, 16, 500), (1, 1032, 16, 700), (1, 16, 16, 4096), (2, 2048, 16, 1500)], ids=str)
+def test_infinite_input(oracle_lib, dev, shape, dtype, layout):
+    """An infinite input makes every later state infinite, not NaN, however small the decays' products
+    over many steps get (B and C positive, so no two infinities cancel)."""
+    inp = config0_inputs(*shape, seed=9)
+    for k in ("B", "C", "z"):
+        inp[k] = np.abs(inp[k])
+    inp["u"][0, 3, 20] = np.inf
+    y, h = gpu_scan(inp, dev, dtype, softplus=True, layout=layout)
+    sub = {k: v[:1, 3:4] if v.ndim == 3 and k in ("u", "delta", "z") else v[:1] if v.ndim == 3 else v[3:4]
+           for k, v in inp.items()}
+    yo, ho = oracle_scan(oracle_lib, sub, dtype, softplus=True)
+    assert np.isinf(yo[0, 0, 20:]).all() and np.isinf(ho).all()
+    assert np.array_equal(y[0, 3] == np.inf, yo[0, 0] == np.inf) and np.array_equal(h[0, 3], ho[0, 0])
+    keep = np.ones(y.shape, bool)
+    keep[0, 3] = False
+    assert np.isfinite(y[keep]).all() and np.isfinite(y[0, 3, :20]).all()
