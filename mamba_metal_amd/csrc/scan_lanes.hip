@@ -315,7 +315,10 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
   if (!SUM && unit == 0 && tid == 0) p.ctl[1] = 0;  // the call's status
 
   // lane n holds the channel's A[n] and the carried state n
-  const float Al = lane < p.dstate ? p.A[c * p.As0 + lane * p.As1] : 0.0f;
+  float Al = lane < p.dstate ? p.A[c * p.As0 + lane * p.As1] : 0.0f;
+  // A = -inf keeps no state from step to step; over steps past the sequence's end and between
+  // neighbouring segments (delta2 0) it would be NaN
+  Al = Al == -__builtin_inff() ? -__FLT_MAX__ : Al;
   const bool mine = SW == 1 || lane % kNG / kStates == part;  // whether this wave has state n = lane
   const bool Apos = __any(Al > 0.0f);
   const bool may_grow = Apos || p.softplus_cut != p.softplus_cut;

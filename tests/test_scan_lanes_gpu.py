@@ -140,3 +140,14 @@ def test_infinite_input(oracle_lib, dev, shape, dtype, layout):
     keep = np.ones(y.shape, bool)
     keep[0, 3] = False
     assert np.isfinite(y[keep]).all() and np.isfinite(y[0, 3, :20]).all()
+
+
+@pytest.mark.parametrize("layout", ["bdl", "bld"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 16, 16, 500), (1, 1032, 16, 700), (1, 16, 16, 4095)], ids=str)
+def test_infinite_decay(oracle_lib, dev, shape, dtype, layout):
+    """A = -inf: a state of its last input alone, also where the sequence ends inside a chunk and from
+    segment to segment."""
+    inp = config0_inputs(*shape, seed=10)
+    inp["A"][:, 7] = inp["A"][:, 15] = -np.inf
+    check(oracle_lib, dev, inp, f"A = -inf {shape}", dtype=dtype, softplus=True, layout=layout)
