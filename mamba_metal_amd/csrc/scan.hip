@@ -1170,6 +1170,18 @@ size_t mm_selective_scan_workspace_size(int64_t batch, int64_t dim, int64_t dsta
   return ws_layout(batch, dim, groups, spl, std::max<int64_t>(seqlen, 1)).total;
 }
 
+// Host only, for the tests (not in the header): the way a valid call with this much workspace
+// goes, as the waves per channel of the scan with time across the lanes (0: scan_kernel) and
+// its time segments.
+int mm_scan_route(const mm_scan_params* a, int32_t* segments) {
+  using namespace mm::scan;
+  int groups = 8, spl = 2, sw = 0;
+  pick_shape(a->dstate, &groups, &spl);
+  const WsLayout w = ws_layout(a->batch, a->dim, groups, spl, std::max<int64_t>(a->seqlen, 1));
+  *segments = mm::lscan::segments(a, a->workspace_bytes >= w.total ? w.total - w.sum : 0, &sw);
+  return sw;
+}
+
 int mm_selective_scan_fwd_strided(const mm_scan_params* a, void* stream) {
   mm::clear_error();
   return mm::scan::fwd(a, stream, false);

@@ -29,6 +29,8 @@ namespace lscan {
 // workspace's sum_bytes for segment summaries (none: time is not split).
 bool preferred(const mm_scan_params* a, size_t sum_bytes);
 int launch(const mm_scan_params* a, int* ctl, float* sum, size_t sum_bytes, void* stream);
+// How it would run: time segments, and the waves per channel (0: scan.hip has the call).
+int segments(const mm_scan_params* a, size_t sum_bytes, int* sw);
 
 }  // namespace lscan
 }  // namespace mm

@@ -34,7 +34,7 @@ constexpr int kTL = 8;                 // steps per lane and chunk
 constexpr int kChunk = 64 * kTL;       // steps per chunk
 constexpr int kNG = 8;                 // states of B and C staged at a time
 constexpr int kItems = kNG * kChunk / 8;  // 8-element items of a staged tensor
-constexpr int kXcds = 8;
+constexpr int kXcds = 8, kCus = 256;
 constexpr int kMaxSeg = 64;  // a wave folds its segment's predecessors, one per lane
 
 // kTime: u, delta, z, y and B, C contiguous along time.  kRows: u, delta, z, y contiguous along
@@ -694,24 +694,31 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
 struct Plan {
   int layout, sw, nseg;
 };
+// Channels of a workgroup: eight waves in all.
+inline int channels_of(int layout, int sw) { return layout == kTime && sw == 4 ? 2 : sw == 2 ? 4 : 8; }
 
 // Which calls: unit strides along one axis, B and C in x's type (anything else keeps scan.hip's
-// packed B/C), and few enough channels.  Measured (us, fp16 unless said, dstate 16, scan.hip
-// against this):
-//   2 to 8 thousand channels: 4x2048x2048 (B x D x L) 125 -> 101 along time, 138 -> 114 along
-//     channels; 4x1536x8192 351 -> 293 and 404 -> 351; 1x2048x2048 48 -> 37 and 53 -> 45.  Above,
-//     scan.hip's chains fill the chip: 4x3072x2048 137 against 145 along time; by rows equal
-//     at 12 thousand (160, 164) and ahead at 10 (4x2560x2048 170 -> 141).  Steps padded to whole
-//     chunks count as work: 4x1536x300 31 against 36.
-//   dstate > 16, where scan.hip has only 64-channel blocks: 2x1536x2048 at 32 states 347 -> 90,
-//     4x3072x2048 469 -> 263, at 40 thousand channels 345 against 424.
-//   fewer: one chunk always (1x1536x512 22 -> 12).  Long sequences on 512 to 1536 channels
-//     keep scan.hip's split over time, whose two passes take fewer slots (1x1024x32768 247
-//     against 292 here), up to lengths where one unsplit pass wins: 1x1536x2048 37 -> 35 and 44 ->
-//     43, 1x1024x2048 29 -> 25 and 32 against 38.  fp32 pays twice for its exponentials there:
-//     1x1024x8192 132 -> 116 along time.
-//   a few hundred and less: both passes here are short (1x16x32768 fp32 109 -> 21, 1x64x8192 37
-//     -> 18); 1x256x32768 93 against 104.
+// packed B/C), and few enough channels.  The lines below are where scan.hip's time and this one's
+// cross, measured over 8 to 16384 channels, 8 to 65536 steps, 1 to 64 states, fp16 and fp32,
+// along time and by rows; of 15549 calls that come here (drawn and large ones, in all types) 7 are
+// slower than scan.hip by 3% or more (14% at most), and they take 0.36 of its time on average.  us, scan.hip's
+// first, fp16 and 16 states unless said, batch x channels x steps:
+//   - A chunk costs the same for 1 or 512 steps, and a launch as many rounds of a workgroup per CU as
+//     it has begun: `waste` is the work done over the work asked for.  One chunk nearly always
+//     pays (1x1536x512 20 -> 12, 1x1024x64 13 -> 9.4), more of them while the waste is small:
+//     1x2560x896 (1.4) 30 -> 28, 1x2560x768 (1.6) 25 -> 28; 1x2048x1152 (1.3) 31 -> 27, 1x2560x1152 (1.6)
+//     32 -> 39; 1x3072x2304 (1.1) 69 -> 60, 1x2560x2304 (1.3) 51 -> 60; by rows 1x2560x896 (1.8) 0.83 of the
+//     time, 1x2560x768 (2.1) 1.12.  Rows of a length that scan.hip cannot load as vectors cost it
+//     a third (1x2560x3001 92 -> 73), and few states cost this kernel less, and scan.hip no less.
+//   - Up to 8 thousand channels (16-bit rows 10): 4x2048x2048 116 -> 96, 4x1536x8192 335 -> 289.  Above,
+//     scan.hip's chains fill the chip.
+//   - Few channels and long: time is split, in two launches (1x16x32768 90 -> 14, 1x64x8192 36 ->
+//     17, 1x256x2048 22 -> 17; 1x256x4608 29 -> 33, 1x512x1280 21 -> 23).  Between these and 2048 (fp32
+//     1024) channels, long sequences keep scan.hip's split, which takes fewer slots (1x1024x32768 247
+//     against 292).
+//   - dstate > 16, where scan.hip has 64-channel blocks of 32 or 64 states that walk all of time: any length,
+//     without a split (1x16x65536 at 32 states in 0.07 of the time), until those blocks fill the chip with
+//     states that are no padding: 1x16384x1024 at 32 and 64 states 0.9 to 1.1 of the time, at 24 and 48 0.5 to 0.8.
 inline Plan plan(const mm_scan_params* a, size_t sum_bytes) {
   Plan pl = {kTime, 0, 1};
   const int64_t ch = a->batch * a->dim, L = a->seqlen;
@@ -728,28 +735,28 @@ inline Plan plan(const mm_scan_params* a, size_t sum_bytes) {
   const bool f32 = a->x_dtype == MM_F32;
   const int64_t nch = ceil_div(L, kChunk);
 
-  const int64_t most = a->dstate > 16 ? 16384 : time_c || f32 ? 8192 : 10240;
+  int64_t most = time_c || f32 ? 8192 : 10240;
+  if (a->dstate > 16)
+    most = ceil_div(a->dstate, 8) % 4 != 0 ? 16384 : ch > 2048 && L <= 256 ? 12288 : ch > 6144 ? 14200 : 16384;
   if (ch * nch * kChunk > most * L) return pl;
+  const bool low = a->dstate <= (f32 ? 4 : 8);
   bool split = false;
-  if (a->dstate > 16) {
-    split = ch <= 512 && nch > 2;
-  } else if (nch == 1) {
-  } else if (time_c) {
-    if (ch >= (f32 ? 1024 : 2048)) {
-    } else if (ch >= 512 && nch <= (ch >= 768 ? 4 : 2)) {
-    } else if ((ch <= 512 && ch * nch <= 2048) || (ch <= 256 && ch * nch <= 4096)) {
-      split = nch > 2;
-    } else {
-      return pl;
-    }
-  } else {
-    if (ch >= 3072 || (ch >= (f32 ? 1024 : 2048) && nch <= 8)) {
-    } else if (ch >= 1536 && nch <= 4) {
-    } else if (ch >= 768 && nch <= 2) {
-    } else if (ch <= 256 && nch >= 4 && ch * nch <= 4096) {
+  if (a->dstate <= 16) {
+    const int64_t w = low ? 2 : 1;
+    const bool few = (ch <= 256 * w && nch <= 4) || (ch <= 192 * w && ch * nch <= 2048) || (ch <= 128 * w && ch * nch <= 4096);
+    const bool some = a->dstate > 4 && a->dstate <= 8;  // one state per lane of scan.hip's, and not few of them
+    if (time_c) {
+      if (nch > 2 && ch < (f32 && nch <= (some ? 16 : 32) ? 1024 : f32 || nch <= 16 || low ? 2048 : 4096) && !(ch >= 768 && nch <= 4)) {
+        if (!few) return pl;
+        split = true;
+      }
+    } else if (f32 && some && nch > 16) {
+      if (!few) return pl;
       split = true;
-    } else {
-      return pl;
+    } else if (nch > 1 && ch < 3072 && !(ch >= (f32 ? 1024 : 2048) && nch <= 8) && !(ch >= 1536 && nch <= 4) &&
+               !(ch >= 768 && nch <= 2)) {
+      if (!few || nch < 4) return pl;
+      split = true;
     }
   }
 
@@ -760,23 +767,44 @@ inline Plan plan(const mm_scan_params* a, size_t sum_bytes) {
   // -> 14.3, 1x2048x1536 40.8 and 41.2, 4x2048x1536 88 and 107; fp32 1x2048x1536 71 -> 55,
   // 1x2048x3072 108 -> 82, 4x2048x1536 165 -> 147 (two waves on eight channels: 20.7, 19.5, 42.6,
   // 121; 57, 109, 166).  Split, as long as the segments leave room.
-  const int64_t seg = std::min<int64_t>(nch, kMaxSeg);
   if (split) {
-    const int64_t bytes = 4 * ch * (a->dstate + 1);
-    int64_t nseg = std::min<int64_t>({seg, static_cast<int64_t>(sum_bytes) / bytes, std::max<int64_t>(1, 4096 / ch)});
+    const int64_t seg = std::min<int64_t>(nch, kMaxSeg), bytes = 4 * ch * (a->dstate + 1);
+    // (without room for summaries one pass over all chunks is still the faster one)
+    const int64_t nseg = std::min<int64_t>({seg, static_cast<int64_t>(sum_bytes) / bytes, std::max<int64_t>(1, 4096 / ch)});
     if (nseg > 1) {
       const int64_t per = ceil_div(nch, nseg);
       pl.nseg = static_cast<int>(ceil_div(nch, per));
     }
     const int64_t w = ch * pl.nseg;
     pl.sw = time_c ? (w <= 1024 ? 4 : w <= 2048 ? 2 : 1) : (w <= 2048 ? 2 : 1);
-  } else {
-    pl.sw = time_c ? (ch <= 1536 ? 4 : ch < 4096 ? 2 : 1) : (f32 || ch <= 1024 ? 2 : 1);
+    return pl;
+  }
+  pl.sw = time_c ? (ch <= 1536 ? 4 : ch < 4096 ? 2 : 1) : (f32 || ch <= 1024 ? 2 : 1);
+  if (a->dstate <= 16 && ch > 1024 && !(nch <= 2 && ch <= 2048 && (nch == 2 || !time_c))) {
+    const int64_t wgs = a->batch * ceil_div(a->dim, channels_of(pl.layout, pl.sw));
+    const double waste = static_cast<double>(nch * kChunk) / L * round_up(wgs, kCus) / wgs;
+    double limit;
+    if (nch == 1) limit = ch <= 3072 ? 5.0 : time_c && f32 && ch > 4096 ? 1.5 : 2.5;
+    else if (low && ch >= 4096 && time_c) limit = 5.0;
+    else if (time_c && nch == 2) limit = 1.45;
+    else if (time_c && f32) limit = nch <= 4 ? 1.45 : ch >= 2048 ? 1.25 : 1.19;
+    else if (time_c) limit = ch <= 1536 ? 1.1 : nch == 3 ? 1.4 : nch == 4 ? 1.33 : ch < 4096 ? 1.1 : 1.19;
+    else if (f32) limit = nch == 2 ? 1.5 : nch == 3 ? 1.4 : nch == 4 && ch < 2048 ? 1.9 : 1.3;
+    else limit = nch == 2 ? 1.95 : nch <= 4 ? 1.5 : 1.25;
+    if (low && (nch <= 8 || (f32 && ch > 1536))) limit *= 1.1;
+    if (time_c && L % 4 != 0) limit *= 1.3;
+    if (waste > limit) pl.sw = 0;
   }
   return pl;
 }
 
 bool preferred(const mm_scan_params* a, size_t sum_bytes) { return plan(a, sum_bytes).sw > 0; }
+
+int segments(const mm_scan_params* a, size_t sum_bytes, int* sw) {
+  const Plan pl = plan(a, sum_bytes);
+  *sw = pl.sw;
+  return pl.nseg;
+}
 
 template <int DT, int LAYOUT, int CH, int SW, bool PAIR = false>
 void launch_n(const Params& p, int64_t batch, hipStream_t s) {
@@ -797,7 +825,7 @@ void launch_dt(const Params& p, int64_t batch, const Plan& pl, hipStream_t s) {
     // 16-bit, unsplit, at most a workgroup per CU: states in pairs (fp32's longer decays keep a SIMD's
     // two waves busy: 1x1000x1024 19.7 and 19.6 us, 2x2048x3072 155 and 203)
     if constexpr (DT != MM_F32) {
-      if (p.nseg == 1 && ceil_div(p.dim, pl.sw == 2 ? 4 : 8) * batch <= 256) {
+      if (p.nseg == 1 && ceil_div(p.dim, channels_of(kRows, pl.sw)) * batch <= kCus) {
         if (pl.sw == 2) launch_n<DT, kRows, 4, 2, true>(p, batch, s);
         else launch_n<DT, kRows, 8, 1, true>(p, batch, s);
         return;

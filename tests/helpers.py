@@ -111,3 +111,30 @@ def check_greedy(got, gpu_logits, ref_logits, n, what, max_exempt_frac=0.05, tol
     print(f"[greedy] {what}: max logit error {err:.2e}; {len(exempt)} of {total} argmax checks "
           f"exempt (oracle top-2 margin <= {2 * err:.2e}): {exempt}")
     assert len(exempt) <= max_exempt_frac * total
+
+
+def scan_route(layout, dtype, batch, dim, dstate, seqlen, workspace_bytes=None, bc_dtype=None):
+    """(waves per channel of the scan with time across the lanes, 0 for the general kernel; time segments)
+    of a call on contiguous (batch, dim, seqlen) ("bdl") or (batch, seqlen, dim) ("bld") tensors.  Host only."""
+    import ctypes
+
+    from mamba_metal_amd import _lib
+
+    lib = _lib.load()
+    p = _lib.ScanParams()
+    p.batch, p.dim, p.dstate, p.seqlen = batch, dim, dstate, seqlen
+
+    def strides(n):
+        return _lib._i64a3(n * seqlen, *((seqlen, 1) if layout == "bdl" else (1, n)))
+
+    for k in ("u", "delta", "z", "y"):
+        setattr(p, f"{k}_stride", strides(dim))
+    p.B_stride = p.C_stride = strides(dstate)
+    p.x_dtype, p.bc_dtype = _lib.dtype_code(dtype), _lib.dtype_code(bc_dtype or dtype)
+    if workspace_bytes is None:
+        workspace_bytes = lib.mm_selective_scan_workspace_size(batch, dim, dstate, seqlen)
+    p.workspace_bytes = workspace_bytes
+    route = lib.mm_scan_route
+    route.argtypes, route.restype = [ctypes.POINTER(_lib.ScanParams), ctypes.POINTER(ctypes.c_int32)], ctypes.c_int
+    segments = ctypes.c_int32()
+    return route(ctypes.byref(p), ctypes.byref(segments)), segments.value
