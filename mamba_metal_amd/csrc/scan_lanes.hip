@@ -130,7 +130,7 @@ __device__ __forceinline__ void lane_scan(float& P, float& h, float pr, float ph
       "s_nop 1\n\t"
       "v_fmac_f32_dpp %1, %1, %3 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
       "s_nop 1"
-      : "+v"(P), "+v"(h)
+      : "+&v"(P), "+&v"(h)
       : "v"(pr), "v"(ph));
 }
 
