@@ -168,42 +168,34 @@ __device__ __forceinline__ void lane_scan2(float& P0, float& h0, float pr0, floa
 // B and C of NG states of a chunk on their way to LDS rows of fp32, zero past the sequence's
 // end and past the last state: one vector of 8 steps of a state (kTime) or of 8 states of a
 // step (kRows) per thread and tensor.
-
 template <int DT, int LAYOUT, int NT>
 struct Stage {
   using T = typename Ty<DT>::T;
   using V = typename Run<DT, 8>::V;
   using U = typename Run<DT, 8>::U;
   static constexpr int kPer = kChunk / 8;         // kTime: 8-step items of a state
-  static constexpr bool kSplit = NT == 2 * kItems;  // half the threads take B, half C
-  static_assert(NT == kItems || kSplit, "one item of B and of C per thread, or of one of them");
-  V v[kSplit ? 1 : 2];
-  const T* ptr[kSplit ? 1 : 2];  // this thread's item of state group 0 and step 0
-  int64_t sn, st;                // its tensor's strides along states and time (kSplit)
+  static_assert(NT == kItems, "one item of B and of C per thread");
+  V v[2];           // of B and C
+  const T* ptr[2];  // this thread's item of state group 0 and step 0
 
-  __device__ __forceinline__ int item(int tid) const { return kSplit ? tid & (kItems - 1) : tid; }
+  // (As a call: with tid written out the compiler schedules the fp32 kernels otherwise, 1x1536x2048
+  // 44 -> 47 us.)
+  __device__ __forceinline__ int item(int tid) const { return tid; }
 
   __device__ __forceinline__ void init(const Params& p, int64_t bat, int tid) {
     const T* const pb = static_cast<const T*>(p.B) + bat * p.Bs0;
     const T* const pc = static_cast<const T*>(p.C) + bat * p.Cs0;
     const int i = item(tid);
-    if constexpr (kSplit) {
-      const bool isb = __builtin_amdgcn_readfirstlane(tid) < kItems;  // whole waves
-      sn = isb ? p.Bs1 : p.Cs1;
-      st = isb ? p.Bs2 : p.Cs2;
-      ptr[0] = (isb ? pb : pc) + (LAYOUT == kTime ? (i / kPer) * sn + 8 * (i % kPer) : i * st);
-    } else {
-      ptr[0] = pb + (LAYOUT == kTime ? (i / kPer) * p.Bs1 + 8 * (i % kPer) : i * p.Bs2);
-      ptr[1] = pc + (LAYOUT == kTime ? (i / kPer) * p.Cs1 + 8 * (i % kPer) : i * p.Cs2);
-    }
+    ptr[0] = pb + (LAYOUT == kTime ? (i / kPer) * p.Bs1 + 8 * (i % kPer) : i * p.Bs2);
+    ptr[1] = pc + (LAYOUT == kTime ? (i / kPer) * p.Cs1 + 8 * (i % kPer) : i * p.Cs2);
   }
 
   __device__ __forceinline__ void load(const Params& p, bool with_c, int g0, int t0, int tid) {
     const bool full = t0 + kChunk <= p.seqlen && g0 + kNG <= p.dstate;
 #pragma unroll
-    for (int x = 0; x < (kSplit ? 1 : 2); ++x) {
+    for (int x = 0; x < 2; ++x) {
       if (x == 1 && !with_c) break;
-      const int64_t s1 = kSplit ? sn : x ? p.Cs1 : p.Bs1, s2 = kSplit ? st : x ? p.Cs2 : p.Bs2;
+      const int64_t s1 = x ? p.Cs1 : p.Bs1, s2 = x ? p.Cs2 : p.Bs2;
       int64_t o;
       if constexpr (LAYOUT == kTime) {
         o = g0 * s1 + t0;
@@ -226,8 +218,8 @@ struct Stage {
                                         float (*sb)[kChunk], float (*sc)[kChunk]) const {
     const bool full = t0 + kChunk <= p.seqlen && g0 + kNG <= p.dstate;
 #pragma unroll
-    for (int x = 0; x < (kSplit ? 1 : 2); ++x) {
-      float(*const dst)[kChunk] = kSplit ? (__builtin_amdgcn_readfirstlane(tid) < kItems ? sb : sc) : x ? sc : sb;
+    for (int x = 0; x < 2; ++x) {
+      float(*const dst)[kChunk] = x ? sc : sb;
       if (!with_c && dst == sc) break;
       if constexpr (LAYOUT == kTime) {
         const int n = item(tid) / kPer, t = 8 * (item(tid) % kPer);
