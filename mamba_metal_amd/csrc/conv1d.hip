@@ -65,11 +65,13 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
     run = blockIdx.x / p.ncgb * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   } else {
     const int64_t gid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (gid >= p.nruns * p.ncg) return;
     cg = gid % p.ncg;
     run = gid / p.ncg;
   }
-  if (cg >= p.ncg || run >= p.nruns) return;
-  const int64_t b = run / p.nchunks, chunk = run % p.nchunks;
+  if (UNI && (cg >= p.ncg || run >= p.nruns)) return;
+  const decltype(run) nchunks = p.nchunks;  // (a 32-bit one cost a strided fp32 call 3 to 7%)
+  const int64_t b = run / nchunks, chunk = run % nchunks;
   const int64_t c0 = cg * kCV;
   const int off = W - static_cast<int>(K > 0 ? K : p.width);  // leading zero taps (K == 0)
 
@@ -86,14 +88,18 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
     for (int u = 0; u < U; ++u)
       xr[u] = *reinterpret_cast<const V8*>(xb + (t0 + u < t_end ? t0 + u : t_end - 1) * p.xs1);
   };
-  if constexpr (VEC) {
+  auto load_first = [&]() __attribute__((always_inline)) {
+    if constexpr (VEC) {
 #pragma unroll
-    for (int k = 0; k < W - 1; ++k) {
-      const int64_t t = t_begin - (W - 1) + k;
-      hr[k] = *reinterpret_cast<const V8*>(xb + (t >= 0 ? t : 0) * p.xs1);
+      for (int k = 0; k < W - 1; ++k) {
+        const int64_t t = t_begin - (W - 1) + k;
+        hr[k] = *reinterpret_cast<const V8*>(xb + (t >= 0 ? t : 0) * p.xs1);
+      }
+      load_group(t_begin);
     }
-    load_group(t_begin);
-  }
+  };
+  // (after the taps at widths 2 and 3: fp32 3 x 777 x 2048 14.8 -> 13.7 us and 17.1 -> 15.2)
+  if constexpr (K == 4 || K == 0) load_first();
 
   // Taps (zero-padded at the old end when K == 0) and bias ((dim,) contiguous, w_dtype).
   // Every load is unconditional, from a clamped in-bounds address, and masked afterwards:
@@ -156,6 +162,8 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
     bias[j] = (cin && p.bias != nullptr) ? bias[j] : 0.0f;
   }
 
+  if constexpr (K == 2 || K == 3) load_first();
+
   // Strided path: x[b, t, c0 .. c0 + 7] (t >= 0) element by element; channels past dim read
   // channel 0 and count as zero.
   auto load_x = [&](int64_t t, float v[kCV]) {
@@ -178,8 +186,12 @@ __global__ __launch_bounds__(kBlock) void conv1d_kernel(const Params p) {
     } else {
       load_x(t >= 0 ? t : 0, win[k]);
     }
+  }
 #pragma unroll
-    for (int j = 0; j < kCV; ++j) win[k][j] = t >= 0 ? win[k][j] : 0.0f;
+  for (int k = 0; k < W - 1; ++k) {
+    const bool tin = t_begin - (W - 1) + k >= 0;
+#pragma unroll
+    for (int j = 0; j < kCV; ++j) win[k][j] = tin ? win[k][j] : 0.0f;
   }
 
   for (int64_t t0 = t_begin; t0 < t_end; t0 += U) {
@@ -406,9 +418,12 @@ int mm_causal_conv1d_fwd(const void* x, const void* weight, const void* bias, vo
   // 4 / 8 / 16 / 32 steps: 2 x 1021 x 1024 5.2 / 6.3 / 8.9 / 13.6, 4 x 2048 x 1536 18.2 / 16.3 / 15.7
   // / 16.4, 8 x 1024 x 2048 23.6 / 21.9 / 18.9 / 17.1, 64 x 512 x 5120 179 / 154 / 139 / 140.
   // The flat range spends more per run and wants more waves, and runs of 8 at least: 4 x 2048 x 1032
-  // 14.9 us at 8 steps, 16.0 at 16; 3 x 777 x 1542 17.9 at 8, 22.0 at 4.
-  const int64_t least = p.uni ? kU : 2 * kU, few = p.uni ? 65536 : 131072;
-  int64_t tc = 32;
+  // 14.9 us at 8 steps, 16.0 at 16; so do taps that are not read as vectors (1 x 2048 x 1536 at
+  // width 3 8.2 us at 8 steps, 8.6 at 4, at width 8 20.9 and 27.1).  Strided x: up to 256 steps, each
+  // of a run's loads being a line of its own (64 x 512 x 5120 along time 3.3 ms, 3.5 at 32 steps).
+  const int64_t least = p.uni && p.w_vec ? kU : 2 * kU;
+  const int64_t few = !p.vec_ok ? 262143 : p.uni ? 65536 : 131072;
+  int64_t tc = p.vec_ok ? 32 : 256;
   while (tc > least && batch * p.ncg * ceil_div(seqlen, tc) <= few) tc /= 2;
   p.tc = tc;
   p.nchunks = static_cast<uint32_t>(ceil_div(seqlen, tc));

@@ -298,3 +298,43 @@ def test_causal_conv1d_runs(dev, B, L, D, dtype):
     assert_close(y.float().cpu().numpy(), ref.numpy(), tol, 4e-6, "conv")
     last = torch.cat([torch.zeros(B, 4, D, dtype=dtype), x], 1)[:, -4:].transpose(1, 2)
     assert torch.equal(state.cpu(), last), "conv state"
+
+
+# What the runs above leave out: the other widths (one, a few, a zero-padded window of eight taps), taps of
+# another type than x and in columns, no bias, no activation, x as half of a wider buffer, at an odd channel
+# and along time, each on channel counts that fill whole waves and that do not.
+@pytest.mark.parametrize("dtype,wdtype", [(torch.float32, torch.float32), (torch.float16, torch.float16),
+                                          (torch.bfloat16, torch.float32), (torch.float16, torch.float32)])
+@pytest.mark.parametrize("width", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("D", [512, 1536, 72])
+@pytest.mark.parametrize("kind", ["plain", "half", "odd", "time", "columns"])
+def test_causal_conv1d_forms(dev, D, width, dtype, wdtype, kind):
+    from mamba_metal_amd.conv1d import causal_conv1d
+
+    B, L = 3, 77
+    rng = np.random.default_rng(D + width)
+    r = lambda *s: torch.as_tensor(rng.standard_normal(s).astype(np.float32))
+    x, w, b = r(B, L, D).to(dtype), r(D, width).to(wdtype), r(D).to(wdtype)
+    use_bias, silu = kind != "half", kind != "odd"
+    xg = x.to(dev)
+    if kind == "half":
+        xg = torch.cat([xg, torch.full_like(xg, float("nan"))], -1)[..., :D]
+    elif kind == "odd":
+        xg = torch.cat([torch.full_like(xg[..., :1], float("nan")), xg], -1)[..., 1:]
+    elif kind == "time":
+        xg = xg.transpose(1, 2).contiguous().transpose(1, 2)
+    wg = w.to(dev)
+    if kind == "columns":
+        wg = wg.t().contiguous().t()
+    state = torch.empty((B, D, width), dtype=dtype, device=dev)
+    y = causal_conv1d(xg, wg, b.to(dev) if use_bias else None, apply_silu=silu, conv_state_out=state)
+    xd = torch.cat([torch.zeros(B, width - 1, D), x.float()], 1).double()
+    ref = sum(xd[:, k:k + L] * w.double()[:, k] for k in range(width))
+    ref = ref + b.double() if use_bias else ref
+    ref = torch.nn.functional.silu(ref) if silu else ref
+    # up to eight fp32 fmas (their terms, of magnitude ~1, may cancel) and SiLU on the hardware's exp and
+    # rcp, then the output's half ulp
+    tol = {torch.float32: 4e-6, torch.float16: 2.0 ** -11 + 4e-6, torch.bfloat16: 2.0 ** -8}[dtype]
+    assert_close(y.float().cpu().numpy(), ref.numpy(), tol, 8e-6, "conv")
+    last = torch.cat([torch.zeros(B, width, D, dtype=dtype), x], 1)[:, -width:].transpose(1, 2)
+    assert torch.equal(state.cpu(), last), "conv state"
