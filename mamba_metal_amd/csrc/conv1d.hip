@@ -425,6 +425,9 @@ int mm_causal_conv1d_fwd(const void* x, const void* weight, const void* bias, vo
   const int64_t few = !p.vec_ok ? 262143 : p.uni ? 65536 : 131072;
   int64_t tc = p.vec_ok ? 32 : 256;
   while (tc > least && batch * p.ncg * ceil_div(seqlen, tc) <= few) tc /= 2;
+  // In place: one run per sequence, which reads every step before it writes it (a run's history is
+  // its predecessor's output otherwise).
+  if (out == x) tc = seqlen;
   p.tc = tc;
   p.nchunks = static_cast<uint32_t>(ceil_div(seqlen, tc));
   p.nruns = batch * ceil_div(seqlen, tc);

@@ -338,3 +338,17 @@ def test_causal_conv1d_forms(dev, D, width, dtype, wdtype, kind):
     assert_close(y.float().cpu().numpy(), ref.numpy(), tol, 8e-6, "conv")
     last = torch.cat([torch.zeros(B, width, D, dtype=dtype), x], 1)[:, -width:].transpose(1, 2)
     assert torch.equal(state.cpu(), last), "conv state"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("B,L,D,width", [(1, 7, 512, 4), (2, 200, 520, 4), (1, 70, 30, 3), (1, 40, 512, 8)])
+def test_causal_conv1d_in_place(dev, B, L, D, width, dtype):
+    """out = x: every step is read before it is written, however many runs a sequence would be cut into."""
+    from mamba_metal_amd.conv1d import causal_conv1d
+
+    g = torch.Generator(device=dev)
+    g.manual_seed(L)
+    x = torch.randn((B, L, D), generator=g, device=dev).to(dtype)
+    w, b = torch.randn((D, 1, width), generator=g, device=dev).to(dtype), torch.randn(D, generator=g, device=dev).to(dtype)
+    ref = causal_conv1d(x, w, b)
+    assert torch.equal(causal_conv1d(x, w, b, out=x), ref)
