@@ -22,7 +22,8 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import (assert_close, config0_inputs, features_inputs, fp16_inputs, plain_inputs)
+from helpers import (assert_close, config0_inputs, features_inputs, fp16_inputs, plain_inputs,
+                     scan_route)
 
 pytestmark = pytest.mark.gpu
 
@@ -483,25 +484,29 @@ def test_edges_against_golden(dev):
 
 def test_handoff_timeout_is_reported_and_bounded(dev):
     """Failure handling of the chained scan's segment hand-off, forced from the host: with
-    a 1-microsecond bound (every real predecessor segment takes far longer) the waits give
+    a 1-microsecond bound the waits give
     up, the kernel still exits, and the status word carries the timeout bit; the same call
     with the default bound then completes with a clear status and the oracle's result
-    (one channel of every block).  640 chains of 32 channels, several segments each."""
+    (one channel of every 32).  192 chains of 48 channels and 8 states, four segments each, on 512
+    resident workgroups: over 300 of them start on a second or third segment at once and wait for
+    the whole of the one before it (64 tiles, tens of microseconds).  (With more chains than
+    workgroups a unit's predecessor is claimed a whole round earlier, and no wait need last.)"""
     from mamba_metal_amd import _lib
     from mamba_metal_amd.selective_scan import (reset_scan_status, scan_status,
                                                 selective_scan_into)
 
     import time
 
-    batch, dim, seqlen = 4, 5120, 8192
+    batch, dim, n, seqlen = 1, 9216, 8, 8192
+    assert scan_route("bdl", torch.float16, batch, dim, n, seqlen)[0] == 0
     g = torch.Generator(device=dev)
     g.manual_seed(5)
     f16 = torch.float16
     u = torch.randn((batch, dim, seqlen), generator=g, device=dev).to(f16)
     d = (torch.randn((batch, dim, seqlen), generator=g, device=dev) * 0.5 - 1.0).to(f16)
-    B = torch.randn((batch, 16, seqlen), generator=g, device=dev).to(f16)
-    C = torch.randn((batch, 16, seqlen), generator=g, device=dev).to(f16)
-    A = -torch.arange(1, 17, device=dev, dtype=torch.float32).expand(dim, 16).contiguous()
+    B = torch.randn((batch, n, seqlen), generator=g, device=dev).to(f16)
+    C = torch.randn((batch, n, seqlen), generator=g, device=dev).to(f16)
+    A = -torch.arange(1, n + 1, device=dev, dtype=torch.float32).expand(dim, n).contiguous()
     y = torch.empty_like(u)
     reset_scan_status(dev)
     t0 = time.perf_counter()
@@ -518,7 +523,7 @@ def test_handoff_timeout_is_reported_and_bounded(dev):
 
     rng = np.random.default_rng(5)
     chans = np.minimum(np.arange(dim // 32) * 32 + rng.integers(0, 32, dim // 32), dim - 1)
-    b = 2
+    b = 0
     uu, dd = u[b, chans].float().cpu().numpy()[None], d[b, chans].float().cpu().numpy()[None]
     yr, _ = cscan.selective_scan(uu, dd, A[chans].cpu().numpy(), B[b:b + 1].float().cpu().numpy(),
                                  C[b:b + 1].float().cpu().numpy(), delta_softplus=True)
