@@ -150,19 +150,28 @@ def test_edge_dstate(oracle_lib, dev, N):
     check(oracle_lib, dev, features_inputs(2, 5, N, 200, seed=N), f"N={N}", softplus=True)
 
 
+@pytest.mark.parametrize("N", [3, 9, 16, 17, 32, 33, 64])
+def test_edge_dstate_general(oracle_lib, dev, N):
+    """The same on the general kernel (strided tensors), at the ends of each count of states per lane."""
+    check(oracle_lib, dev, features_inputs(2, 5, N, 200, seed=N), f"N={N}", softplus=True, layout="gather")
+
+
 @pytest.mark.parametrize("N", [4, 8, 16, 24, 64])
 def test_dstate_many_chains(oracle_lib, dev, N):
     """dstate shapes on the chained path with many channel blocks (2 x 4160 channels: 130
-    64-channel blocks, past the split mode's 128): 32-channel blocks with 1 or 2 states per
-    lane for N <= 16, 64-channel blocks with 8 or 16 for larger N; 4160 = 130 x 32, and a
-    300-step sequence ends inside a tile.  y is a sum of N terms C[n]*h[n] of magnitude ~2-4
+    64-channel blocks, past the split mode's 128; for N > 16 2 x 8224, past what the lane scan
+    takes): 32-channel blocks with 1 or 2 states per
+    lane for N <= 16, 64-channel blocks with 8 or 16 for larger N; 4160 = 130 x 32 (8224 leaves a half
+    block), and a 300-step sequence ends inside a tile.  y is a sum of N terms C[n]*h[n] of magnitude ~2-4
     that largely cancel, so its fp32 rounding grows with N (over these 2.5 M outputs the
     worst N = 64 element was 6.1e-5 off at |y| = 0.86).  The bar is therefore set by a
     plain fp32 evaluation of the same recurrence (the C oracle in fp32, libm expf): y's
     absolute bar is the larger of 1e-5 and twice the fp32 oracle's own worst error against
     the fp64 one on these inputs, so the kernel must be no worse than that; the states keep
     the plain 1e-5 bar."""
-    inp = features_inputs(2, 4160, N, 300, seed=100 + N)
+    dim = 4160 if N <= 16 else 8224
+    assert scan_route("bdl", torch.float32, 2, dim, N, 300)[0] == 0
+    inp = features_inputs(2, dim, N, 300, seed=100 + N)
     yg, hg = gpu_scan(inp, dev, torch.float32, None, True, True, True)
     yo, ho = oracle_scan(oracle_lib, inp, torch.float32, None, True, True, True)
     y32, _ = oracle_scan(oracle_lib, inp, torch.float32, None, True, True, True, precision="f32")
@@ -191,9 +200,10 @@ def test_empty_and_state_only(dev):
 # --- layouts and dtypes ------------------------------------------------------
 @pytest.mark.parametrize("layout", ["bld", "gather"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
-def test_layouts(oracle_lib, dev, layout, dtype):
-    inp = config0_inputs(2, 64, 16, 256, seed=5) if dtype == torch.float32 else \
-        fp16_inputs(2, 64, 16, 256, seed=5)
+@pytest.mark.parametrize("n", [16, 12])  # 12 states by rows: the general kernel (its channel-contiguous loads)
+def test_layouts(oracle_lib, dev, layout, dtype, n):
+    inp = config0_inputs(2, 64, n, 256, seed=5) if dtype == torch.float32 else \
+        fp16_inputs(2, 64, n, 256, seed=5)
     check(oracle_lib, dev, inp, f"layout {layout}", dtype=dtype, softplus=True, layout=layout)
 
 
@@ -252,9 +262,12 @@ def test_channel_contiguous_views_keep_their_layout(oracle_lib, dev):
     assert_close(h.cpu().numpy(), ho, 1e-3, 1e-3, "channel-contiguous state")
 
 
-def test_unaligned_seqlen_uses_gather_path(oracle_lib, dev):
-    # L % 8 != 0 disables the 16-byte vector path for the (batch, dim, seqlen) layout.
-    check(oracle_lib, dev, fp16_inputs(2, 40, 16, 101, seed=6), "L=101 fp16", dtype=torch.float16,
+@pytest.mark.parametrize("dim", [40, 4160])
+def test_unaligned_seqlen_uses_gather_path(oracle_lib, dev, dim):
+    # L % 8 != 0 disables the 16-byte vector path for the (batch, dim, seqlen) layout (of the general
+    # kernel, which has the 4160 channels; 40 run on the lane scan).
+    assert (scan_route("bdl", torch.float16, 2, dim, 16, 101)[0] == 0) == (dim == 4160)
+    check(oracle_lib, dev, fp16_inputs(2, dim, 16, 101, seed=6), "L=101 fp16", dtype=torch.float16,
           softplus=True)
 
 
@@ -327,6 +340,7 @@ def _blockwise_parity(oracle_lib, dev, batch, dim, seqlen, seed, dtype=torch.flo
     g = torch.Generator(device=dev)
     g.manual_seed(seed)
     f16 = dtype
+    assert scan_route("bdl", dtype, batch, dim, 16, seqlen)[0] == 0
     u = torch.randn((batch, dim, seqlen), generator=g, device=dev, dtype=torch.float32).to(f16)
     d = (torch.randn((batch, dim, seqlen), generator=g, device=dev) * 0.5 - 1.0).to(f16)
     z = torch.randn((batch, dim, seqlen), generator=g, device=dev).to(f16)
@@ -361,9 +375,9 @@ def _blockwise_parity(oracle_lib, dev, batch, dim, seqlen, seed, dtype=torch.flo
 
 
 def test_split_mode_matches_chained(oracle_lib, dev):
-    """Few channel chains take the split path (segment summaries, then every segment from
-    the folded carry); many take the chained path.  A slice of a chained-mode call, rerun
-    alone, goes split: each must match the fp64 oracle at the fp32 bar, so the two lie
+    """Some hundred channels take the split path (segment summaries, then every segment from
+    the folded carry; fewer run on the lane scan); many take the chained path.  A slice of a
+    chained-mode call, rerun alone, goes split: each must match the fp64 oracle at the fp32 bar, so the two lie
     within twice that of each other.  A spans [-2, -0.001] with delta <= 0.1 and no
     softplus, so the slowest states carry across many 128-step segments (checked below)."""
     from mamba_metal_amd import selective_scan
@@ -379,11 +393,14 @@ def test_split_mode_matches_chained(oracle_lib, dev):
     A = -(torch.rand((dim, n), generator=g, device=dev) * 1.999 + 0.001)
     D = torch.randn(dim, generator=g, device=dev)
     y, h = selective_scan(u, d, A, B, C, D=D, z=z, return_state=True)
-    b, c0, c1 = 1, 64, 192                   # 2 channel blocks: split
+    b, c0, c1 = 1, 64, 192                   # checked: 2 of the 10 channel blocks of a split call
+    assert scan_route("bdl", torch.float32, batch, dim, n, L)[0] == scan_route("bdl", torch.float32, 1, 640, n, L)[0] == 0
+    few = lambda t: t[b:b + 1, c0:c0 + 640].contiguous()
     sl = lambda t: t[b:b + 1, c0:c1].contiguous()
-    ys, hs = selective_scan(sl(u), sl(d), A[c0:c1].contiguous(), B[b:b + 1].contiguous(),
-                            C[b:b + 1].contiguous(), D=D[c0:c1].contiguous(), z=sl(z),
+    ys, hs = selective_scan(few(u), few(d), A[c0:c0 + 640].contiguous(), B[b:b + 1].contiguous(),
+                            C[b:b + 1].contiguous(), D=D[c0:c0 + 640].contiguous(), z=few(z),
                             return_state=True)
+    ys, hs = ys[:, :c1 - c0], hs[:, :c1 - c0]
     torch.cuda.synchronize()
     cpu = lambda t: t.cpu().numpy()
     yo, ho = oracle_lib.selective_scan(cpu(sl(u)), cpu(sl(d)), cpu(A[c0:c1]), cpu(B[b:b + 1]),
@@ -401,8 +418,10 @@ def test_split_mode_matches_chained(oracle_lib, dev):
     assert (y0 - ys[..., -128:]).abs().max().item() > 0.1
 
 
-def test_split_lone_chain_many_segments(oracle_lib, dev):
-    """The reference's benchmark shape (B=1, D=16, N=16, L=32768; one chain) splits into
+@pytest.mark.parametrize("bc_dtype,lanes", [(torch.float32, (4, 64)), (torch.float16, (0, 1))])
+def test_split_lone_chain_many_segments(oracle_lib, dev, bc_dtype, lanes):
+    """The reference's benchmark shape (B=1, D=16, N=16, L=32768): 64 segments on the lane scan; with B
+    and C in another type one chain of the general kernel, which splits into
     up to 256 segments, so the last segment folds 255 summaries.  Slow decay (A in
     [-2, -0.001], delta <= 0.1) keeps states alive across many segments; fp32 bar against
     the fp64 oracle, y and final state."""
@@ -413,13 +432,14 @@ def test_split_lone_chain_many_segments(oracle_lib, dev):
     batch, dim, n, L = 1, 16, 16, 32768
     u = torch.randn((batch, dim, L), generator=g, device=dev)
     d = torch.rand((batch, dim, L), generator=g, device=dev) * 0.09 + 0.01
-    B = torch.randn((batch, n, L), generator=g, device=dev)
-    C = torch.randn((batch, n, L), generator=g, device=dev)
+    B = torch.randn((batch, n, L), generator=g, device=dev).to(bc_dtype)
+    C = torch.randn((batch, n, L), generator=g, device=dev).to(bc_dtype)
     A = -(torch.rand((dim, n), generator=g, device=dev) * 1.999 + 0.001)
+    assert scan_route("bdl", torch.float32, batch, dim, n, L, bc_dtype=bc_dtype) == lanes
     y, h = selective_scan(u, d, A, B, C, return_state=True)
     torch.cuda.synchronize()
     cpu = lambda t: t.cpu().numpy()
-    yo, ho = oracle_lib.selective_scan(cpu(u), cpu(d), cpu(A), cpu(B), cpu(C))
+    yo, ho = oracle_lib.selective_scan(cpu(u), cpu(d), cpu(A), cpu(B.float()), cpu(C.float()))
     assert_close(cpu(y), yo, 1e-5, 1e-5, "lone chain y")
     assert_close(cpu(h), ho, 1e-5, 1e-5, "lone chain state")
 
