@@ -17,6 +17,8 @@ import numpy as np
 import pytest
 import torch
 
+from helpers import scan_route
+
 pytestmark = pytest.mark.gpu
 
 
@@ -94,10 +96,12 @@ def test_noalloc_matches_workspace_entry_point(dev):
 
     lib = _lib.load()
     # (4, 5120, 2048): 320 channel chains, chained segment hand-offs through the static
-    # array; (3, 1000, 5000): 48 chains, the split mode's segment summaries; then a
-    # smaller call on the same array
+    # array; (1, 640, 9000): 20 chains, the split mode's segment summaries; the lane scan in one
+    # launch and with its segments' summaries; then a smaller call on the same array
     status = torch.zeros(1, dtype=torch.int32, device=dev)
-    for shape, seed in (((4, 5120, 2048), 1), ((3, 1000, 5000), 2), ((1, 200, 700), 3)):
+    for shape, seed, route in (((4, 5120, 2048), 1, (0, 1)), ((1, 640, 9000), 4, (0, 1)), ((3, 1000, 5000), 2, (2, 1)),
+                               ((1, 16, 8192), 5, (4, 16)), ((1, 200, 700), 3, (4, 1))):
+        assert scan_route("bdl", torch.float16, shape[0], shape[1], 16, shape[2]) == route
         ins = _inputs(dev, *shape, seed)
         need = lib.mm_selective_scan_workspace_size(shape[0], shape[1], 16, shape[2])
         assert 0 < need <= _lib.SCAN_SCRATCH_BYTES
@@ -137,6 +141,29 @@ def test_noalloc_chained_when_summaries_do_not_fit(dev):
     assert torch.isfinite(y1).all() and torch.isfinite(h1).all()
     assert_close(y1.float().cpu().numpy(), y0.float().cpu().numpy(), 1e-3, 1e-3, "y")
     assert_close(h1.cpu().numpy(), h0.cpu().numpy(), 1e-3, 1e-3, "state")
+
+
+def test_noalloc_lanes_when_summaries_do_not_fit(dev):
+    """B=32, D=2, L=4096: the lane scan's eight segments with the caller's workspace, one pass over
+    eight chunks on the static array: equal at the fp16 bar (the sums in another order)."""
+    from mamba_metal_amd import _lib
+
+    from helpers import assert_close
+
+    lib = _lib.load()
+    shape = (32, 2, 4096)
+    need = lib.mm_selective_scan_workspace_size(shape[0], shape[1], 16, shape[2])
+    assert need > _lib.SCAN_SCRATCH_BYTES
+    assert scan_route("bdl", torch.float16, 32, 2, 16, 4096) == (4, 8)
+    assert scan_route("bdl", torch.float16, 32, 2, 16, 4096, _lib.SCAN_SCRATCH_BYTES) == (4, 1)
+    ins = _inputs(dev, *shape, 6)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    y0, h0 = _call(lib, "fwd", ins, ws)
+    y1, h1 = _call(lib, "noalloc", ins)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y1).all() and torch.isfinite(h1).all()
+    assert_close(y1.float().cpu().numpy(), y0.float().cpu().numpy(), 1e-3, 1e-3, "y")
+    assert_close(h1.cpu().numpy(), h0.cpu().numpy(), 1e-5, 1e-5, "state")  # fp32 state either way
 
 
 def test_noalloc_rejects_oversize(dev):
