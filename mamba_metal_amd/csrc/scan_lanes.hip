@@ -7,18 +7,22 @@
 // computed once and kept in registers; the lane's end state from zero (one fma per step); an
 // inclusive scan of the lanes' (decay, end state) pairs through DPP (a lane's decay is
 // exp2 of A times its sum of delta2, so it is not multiplied up); then the recurrence once more
-// from the lane's true start state, and y += C h.  Seven VALU slots per (channel, state, step)
-// -- one of six more than the sequential walk -- plus ~30 per state and chunk for the lane scan,
-// and y needs no sum over waves.  B and C are staged in LDS as fp32, eight states at a time
+// from the lane's true start state, and y += C h.  Per (channel, state, step) that is seven VALU slots
+// (the sequential walk has six), and per state and chunk ~30 for the lane scan and three more
+// exponentials, which is five more per update over a lane's eight steps; y needs no sum over waves.  B and C are staged in LDS as fp32, eight states at a time
 // (the next group's loads in flight during this one's arithmetic), shared by the workgroup's
 // channels.  SW > 1 shares a channel's states among SW waves, for launches that would leave
 // SIMDs idle; with few channels and a long sequence time is split as well: a first launch
 // (SUM) leaves every segment's end state from zero and its sum of delta2, and the second folds
 // its predecessors' with one more lane scan.
 //
-// What bounds it: VALU issue (at B=4 D=1536 L=4096 fp16, 12 instructions and 13.9 issue slots
-// per update, 98% of the VALU's cycles busy), against 9.6-12 slots for scan.hip where that one's
-// chains fill the chip, and its 14-40 where they do not.  Tried and not kept: 16 steps per
+// What bounds it: VALU issue (at B=4 D=1536 L=4096 along time, counted: fp16 12.1 instructions and 14.0
+// issue slots per update, 90% of the VALU's cycles busy, fp32 27.3, 27.9 and 97%; by rows fp16 12.6, 14.5
+// and 85%), against 9.6-12 slots for scan.hip where that one's
+// chains fill the chip, and its 14-40 where they do not.  The registers allow four waves per SIMD,
+// in fp32 at the price of 8 to 20 of them in scratch (along time on one and two waves per
+// channel, by rows on one).  With a workgroup per CU or less, a chunk's dependent steps and the
+// fetches of code that runs once.  Tried and not kept: 16 steps per
 // lane (11 slots, but two waves per SIMD instead of four: B=4 D=1536 L=4096 149 -> 180 us), two
 // states interleaved per wave where the chip is full (149 -> 186), the next state's LDS reads ahead
 // (149 -> 151), by rows both state groups of B and C loaded together (1x2048x1536 40.8 -> 42.8).
