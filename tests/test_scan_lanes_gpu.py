@@ -136,6 +136,27 @@ def test_growing_states(oracle_lib, dev, layout, shape, quiet):
 
 
 @pytest.mark.parametrize("layout", ["bdl", "bld"])
+@pytest.mark.parametrize("kind", ["a rate above zero", "steps below zero", "both"])
+@pytest.mark.parametrize("shape", [(1, 16, 16, 500), (1, 1032, 16, 700), (1, 16, 16, 4100)], ids=str)
+def test_states_that_grow_a_little(oracle_lib, dev, layout, kind, shape):
+    """Growth far below the products' range, beside decays far beyond it: rates of up to 0.002 (over 4100
+    steps of 0.05, a factor of 1.5) and a few steps of about -0.01 (growth by e^(16 x 0.01) at most each)."""
+    on_lanes(layout, torch.float32, shape)
+    inp = config0_inputs(*shape, seed=11)
+    rng = np.random.default_rng(11)
+    inp["delta"][:] = rng.normal(0.05, 0.02, inp["delta"].shape) if kind != "a rate above zero" else 0.05
+    if kind != "steps below zero":
+        inp["A"] = np.broadcast_to(np.linspace(-16.0, 0.002, shape[2], dtype=np.float32), inp["A"].shape).copy()
+    y, h = gpu_scan(inp, dev, layout=layout)
+    yo, ho = oracle_scan(oracle_lib, inp)
+    # y sums 16 terms that may cancel: the bar of an fp32 evaluation, as in test_dstate_many_chains
+    y32, h32 = oracle_scan(oracle_lib, inp, precision="f32")
+    e = lambda a, b: float(np.abs(a.astype(np.float64) - b).max())
+    assert_close(y, yo, 1e-5, max(1e-5, 2 * e(y32, yo)), "y")
+    assert_close(h, ho, 1e-5, max(1e-5, 2 * e(h32, ho)), "state")
+
+
+@pytest.mark.parametrize("layout", ["bdl", "bld"])
 @pytest.mark.parametrize("L,t", [(500, 130), (2000, 700), (2000, 1999)])
 def test_nan_stays_behind(dev, layout, L, t):
     """A NaN input reaches no earlier step and no other channel."""
