@@ -179,7 +179,7 @@ int mm_selective_scan_fwd_noalloc(const void* u, const void* delta, const float*
  * x/out strides are (batch, time, channel) in elements; weight is (dim, width)
  * with strides w_stride (the HF/torch (dim, 1, width) tensor viewed 2-D).
  * bias and conv_state_out ((batch, dim, width) contiguous, x_dtype) may be NULL.
- * width <= 8. */
+ * out may be x itself (the same strides).  width <= 8. */
 int mm_causal_conv1d_fwd(const void* x, const void* weight, const void* bias, void* out,
                          void* conv_state_out, int64_t batch, int64_t seqlen, int64_t dim,
                          int64_t width, const int64_t x_stride[3], const int64_t out_stride[3],
