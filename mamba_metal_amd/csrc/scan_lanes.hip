@@ -318,16 +318,6 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
   const bool mine = SW == 1 || lane % kNG / kStates == part;  // whether this wave has state n = lane
   const bool Apos = __any(Al > 0.0f);
   const bool may_grow = Apos || p.softplus_cut != p.softplus_cut;
-  float Aup = 0.0f, Adown = 0.0f;  // the largest of the rates above and below zero
-  if (may_grow) {
-    float hi = Al, lo = Al;
-    for (int m = 32; m > 0; m >>= 1) {
-      hi = fmaxf(hi, lane_xor(hi, m));
-      lo = fminf(lo, lane_xor(lo, m));
-    }
-    Aup = lane_value(fmaxf(hi, 0.0f), 0);  // (scalar registers)
-    Adown = lane_value(fmaxf(-lo, 0.0f), 0);
-  }
   float carry = 0.0f;
   float dsum = 0.0f;  // SUM: delta2 over the segment
 
@@ -504,8 +494,8 @@ __global__ __launch_bounds__(64 * CH * SW, PAIR ? 2 : 4) void lane_scan_kernel(c
           float pos = 0.0f, r, hf, all;
 #pragma unroll
           for (int j = 0; j < kTL; ++j) pos += fmaxf(d2[j], 0.0f);
-          prefix(pos, r, hf, all);  // of the steps above zero; those below it: all - Sall
-          serial = !(lane_value(all, 63) * Aup < 60.0f && lane_value(all - Sall, 63) * Adown < 60.0f);
+          prefix(pos, r, hf, all);  // of the steps above zero; those below it: Sall - all
+          serial = __any(!(lane_value(all, 63) * Al < 60.0f && lane_value(Sall - all, 63) * Al < 60.0f));
         }
       }
       if (last) {  // in flight during these states
