@@ -17,8 +17,8 @@
 // its predecessors' with one more lane scan.
 //
 // What bounds it: VALU issue (at B=4 D=1536 L=4096 along time, counted: fp16 12.1 instructions and 14.0
-// issue slots per update, 90% of the VALU's cycles busy, fp32 27.3, 27.9 and 97%; by rows fp16 12.6, 14.5
-// and 85%), against 9.6-12 slots for scan.hip where that one's
+// issue slots per update, 91% of the VALU's cycles busy, fp32 27.3, 27.9 and 95%; by rows fp16 12.6, 14.5
+// and 86%), against 9.6-12 slots for scan.hip where that one's
 // chains fill the chip, and its 14-40 where they do not.  The registers allow four waves per SIMD,
 // in fp32 at the price of 8 to 20 of them in scratch (along time on one and two waves per
 // channel, by rows on one).  With a workgroup per CU or less, a chunk's dependent steps and the
